@@ -674,58 +674,152 @@ __global__ __launch_bounds__(256) void argmax_tiles_kernel(const float* __restri
   }
 }
 
-// fp32 path (parity runs): one wave per output row of W, 16 token rows per workgroup row-block.
-// Lane l sums k = l, l + 64, ... in order, then a fixed xor tree over the 64 lanes.
-template <int EPI>
+// fp32 path (parity runs).  Every output is one wave's: lane l sums k = l, l + 64, ... in order (multiply and add
+// each rounded), then a fixed xor tree over the 64 lanes (32, 16, 8, 4, 2, 1).  Bound by the vector ALU from ~16 rows
+// on (two instructions per product; no FMA, so that the oracle can restate the sums), by the weight stream below.  A
+// wave owns NT weight rows x MB token rows, so one W and one A value of each k step serve NT MB products (a wave per
+// weight row, which loaded 16 A values per W value, ran at a tenth of the vector rate), and the tree is one pass that
+// halves the values at every level instead of one tree per output.  1B layer on MI355X: w13 at 20 / 121 rows
+// 271 / 1205 -> 54 / 270 us, w2 at 121 rows ~1400 -> 129 us (vector floor at 121 rows: 207 and 103 us).
+template <int O, int N>
+__device__ __forceinline__ void f32_tree_level(float (&v)[N], int lane) {
+  // one level of the tree over N values at once: value i of the lower half stays in the lanes with bit O clear and
+  // value i + N / 2 takes the others, both as own + partner's (the additions of the plain xor tree, whose two lanes
+  // of a pair hold the same sum); with one value left, the plain level
+  if constexpr (N == 1) {
+    v[0] += __shfl_xor(v[0], O, 64);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      if constexpr (O >= 16) {
+        // gfx950 row swaps: first result = the pair's lower lanes of both values, second = its upper lanes
+        const uint32_t a = __float_as_uint(v[i]), b = __float_as_uint(v[i + N / 2]);
+        const auto p = O == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false)
+                               : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        v[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      } else {
+        const bool up = (lane & O) != 0;
+        const float keep = up ? v[i + N / 2] : v[i], send = up ? v[i] : v[i + N / 2];
+        v[i] = keep + __shfl_xor(send, O, 64);
+      }
+    }
+  }
+}
+
+template <int O, int N>
+__device__ __forceinline__ float f32_tree(float (&v)[N], int lane) {
+  f32_tree_level<O, N>(v, lane);
+  if constexpr (O == 1) {
+    return v[0];
+  } else {
+    constexpr int H = N > 1 ? N / 2 : 1;
+    float h[H];
+#pragma unroll
+    for (int i = 0; i < H; ++i) h[i] = v[i];
+    return f32_tree<O / 2, H>(h, lane);
+  }
+}
+
+constexpr int f32_pow2(int n) { return n <= 1 ? 1 : (n <= 2 ? 2 : (n <= 4 ? 4 : (n <= 8 ? 8 : 16))); }
+
+template <bool SILU, int NT, int MB>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, long lda,
-                                                       const float* __restrict__ W, long ldw, float* __restrict__ C,
-                                                       long ldc, const float* __restrict__ R, long ldr, int M, int N,
-                                                       int K, int ffn) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + wave;
-  if (n >= N) return;
-  const int m0 = blockIdx.y * 16;
-  const int mc = min(16, M - m0);
-  float acc[16], accu[16];
+                                                       const float* __restrict__ W, long ldw, float* C, long ldc,
+                                                       const float* R, long ldr, int M, int N, int K, int ffn,
+                                                       int n_tiles, int m_tiles) {
+  constexpr int NB = SILU ? NT / 2 : NT;  // output columns per wave (silu-mul: rows n of the gate, ffn + n of the up half)
+  constexpr int MP = f32_pow2(MB);
+  constexpr int NA = NT * MP;             // sums of a wave, padded to a power of two; sum (t, r) at t MP + r
+  static_assert(NA <= 64 && (!SILU || NT % 2 == 0), "one lane per sum");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // token tiles of one row tile 8 launch slots apart (same XCD: its L2 serves the repeated weight reads)
+  int tn = blockIdx.x, tm = 0;
+  if (m_tiles > 1) {
+    const int slot = blockIdx.x >> 3;
+    tm = slot % m_tiles;
+    tn = (slot / m_tiles) * 8 + (blockIdx.x & 7);
+    if (tn >= n_tiles) return;
+  }
+  const int n0 = (tn * 4 + wave) * NB, m0 = tm * MB;
+  if (n0 >= N) return;
+  // rows past the end read the last one; their sums are dropped
+  const float* wr[NT];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = accu[r] = 0.f;
-  const float* wg = W + (long)n * ldw;
-  const float* wu = W + (long)(ffn + n) * ldw;
-  for (int k = lane; k < K; k += 64) {
-    const float wv = wg[k];
-    const float uv = (EPI == LSK_EPI_SILU_MUL) ? wu[k] : 0.f;
+  for (int t = 0; t < NT; ++t) {
+    const int n = min(n0 + (t < NB ? t : t - NB), N - 1);
+    wr[t] = W + (long)(t < NB ? n : ffn + n) * ldw;
+  }
+  const float* ar[MB];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      if (r < mc) {
-        const float a = A[(long)(m0 + r) * lda + k];
-        acc[r] += a * wv;
-        if (EPI == LSK_EPI_SILU_MUL) accu[r] += a * uv;
+  for (int r = 0; r < MB; ++r) ar[r] = A + (long)min(m0 + r, M - 1) * lda;
+  float acc[NT][MB];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < MB; ++r) acc[t][r] = 0.f;
+  auto mac = [&](const float (&w)[NT], const float (&a)[MB]) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < MB; ++r) acc[t][r] += a[r] * w[t];
+  };
+  // weights come UW steps of 64 k at a time, one unit ahead; activations (cached) one step ahead
+  constexpr int UW = 4;
+  const int steps = K / 64, units = steps / UW;
+  float w[2][UW][NT], a[2][MB];
+  auto load_w = [&](float (&x)[UW][NT], int u) {
+#pragma unroll
+    for (int s = 0; s < UW; ++s)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x[s][t] = (wr[t] + (u * UW + s) * 64)[lane];
+  };
+  auto load_a = [&](float (&x)[MB], int s) {
+#pragma unroll
+    for (int r = 0; r < MB; ++r) x[r] = (ar[r] + s * 64)[lane];
+  };
+  if (units > 0) {
+    load_w(w[0], 0);
+    load_a(a[0], 0);
+    for (int u = 0; u < units; u += 2) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (u + h < units) {
+          load_w(w[h ^ 1], min(u + h + 1, units - 1));  // (past the last unit: reloaded, unused)
+#pragma unroll
+          for (int s = 0; s < UW; ++s) {
+            load_a(a[(s + 1) & 1], min((u + h) * UW + s + 1, steps - 1));
+            mac(w[h][s], a[s & 1]);
+          }
+        }
       }
     }
   }
+  for (int s = units * UW; s * 64 < K; ++s) {
+    const int k = s * 64 + lane;
+    if (k < K) {
+      float w1[NT], a1[MB];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+      for (int t = 0; t < NT; ++t) w1[t] = wr[t][k];
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      acc[r] += __shfl_xor(acc[r], o, 64);
-      if (EPI == LSK_EPI_SILU_MUL) accu[r] += __shfl_xor(accu[r], o, 64);
+      for (int r = 0; r < MB; ++r) a1[r] = ar[r][k];
+      mac(w1, a1);
     }
   }
-  if (lane < mc) {
-    float v = 0.f, u = 0.f;
+  float v[NA];
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      if (r == lane) {
-        v = acc[r];
-        u = accu[r];
-      }
-    const int m = m0 + lane;
-    float outv;
-    if (EPI == LSK_EPI_SILU_MUL) outv = silu_f(v) * u;
-    else if (EPI == LSK_EPI_RESIDUAL) outv = R[(long)m * ldr + n] + v;
-    else outv = v;
-    C[(long)m * ldc + n] = outv;
-  }
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < MP; ++r) v[t * MP + r] = r < MB ? acc[t][r < MB ? r : 0] : 0.f;
+  const float sum = f32_tree<32, NA>(v, lane);  // lane l holds sum l / (64 / NA)
+  const float up = SILU ? __shfl_xor(sum, 32, 64) : 0.f;  // (the up rows are the upper half of the sums)
+  const int id = lane / (64 / NA), t = id / MP, r = id - t * MP;
+  const int n = n0 + t, m = m0 + r;
+  if (lane % (64 / NA) != 0 || t >= NB || r >= MB || n >= N || m >= M) return;
+  float outv = sum;
+  if (SILU) outv = silu_f(sum) * up;
+  else if (R != nullptr) outv = R[(long)m * ldr + n] + sum;
+  C[(long)m * ldc + n] = outv;
 }
 
 // ----------------------------------------------------------------------------- weight packing
@@ -1008,6 +1102,47 @@ static int launch_wide(int epi, hipStream_t s, const uint16_t* A, long lda, cons
   return M;
 }
 
+// fp32 tiles: MB token rows x NT weight rows per wave, chosen over the 1B shape's projections at 1-200 rows (MI355X,
+// cold weights).  MB splits M evenly into tiles of at most `cap` rows:
+//   8 rows by default: 1B w2 / o at 121 rows 129 / 35 us (16-row tiles 122 / 35, 4-row tiles 153 / 40);
+//   16 for up to 32 rows of a weight of >= 8192 rows, whose stream from HBM is what a second tile repeats: w13 at 20
+//     rows 54 us (8-row tiles 66);
+//   4 for up to 32 rows where 8-row tiles would give fewer than 2560 waves: qkv at 20 rows 13.3 us (8-row tiles 15.6).
+// NT = 4, or 2 for up to 4 rows of a weight of < 8192 rows, where the wave count limits the stream: w2 at 1 / 4 rows
+// 18.5 / 22.6 us (NT = 4: 21.0 / 28.3).
+template <bool SILU, int NT, int MB>
+static void launch_f32_tile(hipStream_t s, const float* A, long lda, const float* W, long ldw, float* C, long ldc,
+                            const float* R, long ldr, int M, int N, int K, int ffn) {
+  constexpr int cols = 4 * (SILU ? NT / 2 : NT);
+  const int nt = (N + cols - 1) / cols, mt = (M + MB - 1) / MB;
+  const dim3 grid(mt > 1 ? (unsigned)((nt + 7) / 8 * 8 * mt) : (unsigned)nt);
+  gemm_f32_kernel<SILU, NT, MB><<<grid, 256, 0, s>>>(A, lda, W, ldw, C, ldc, R, ldr, M, N, K, ffn, nt, mt);
+}
+
+template <bool SILU>
+static void launch_f32(hipStream_t s, const float* A, long lda, const float* W, long ldw, float* C, long ldc,
+                       const float* R, long ldr, int M, int N, int K, int ffn) {
+  const long rows = (long)(SILU ? 2 : 1) * N;
+  int cap = 8;
+  if (M <= 32 && rows >= 8192) cap = 16;
+  else if (M <= 32 && rows * ((M + 7) / 8) < 4 * 2560) cap = 4;
+  const int tiles = (M + cap - 1) / cap, mb = (M + tiles - 1) / tiles;
+#define LSK_F32(NT_, MB_) launch_f32_tile<SILU, NT_, MB_>(s, A, lda, W, ldw, C, ldc, R, ldr, M, N, K, ffn)
+  if (M <= 4 && rows < 8192) {
+    if (mb <= 1) LSK_F32(2, 1);
+    else if (mb <= 2) LSK_F32(2, 2);
+    else LSK_F32(2, 4);
+  } else if (mb <= 1) LSK_F32(4, 1);
+  else if (mb <= 2) LSK_F32(4, 2);
+  else if (mb <= 4) LSK_F32(4, 4);
+  else if (mb <= 6) LSK_F32(4, 6);
+  else if (mb <= 8) LSK_F32(4, 8);
+  else if (mb <= 10) LSK_F32(4, 10);
+  else if (mb <= 12) LSK_F32(4, 12);
+  else LSK_F32(4, 16);
+#undef LSK_F32
+}
+
 extern "C" int lsk_gemm(int dtype, const void* A, long lda, const void* W, long ldw, void* C, long ldc,
                         const void* R, long ldr, int M, int N, int K, int epilogue, int ffn, void* stream) {
   LSK_REQUIRE(A && W && C, LSK_EARG, "lsk_gemm: null pointer");
@@ -1039,17 +1174,13 @@ extern "C" int lsk_gemm(int dtype, const void* A, long lda, const void* W, long 
     return lsk_check_launch("lsk_gemm(bf16)");
   }
   if (dtype == LSK_DTYPE_F32) {
-    dim3 grid((N + 3) / 4, (M + 15) / 16);
     const float* a = (const float*)A;
     const float* w = (const float*)W;
-    float* c = (float*)C;
-    const float* r = (const float*)R;
-    if (epilogue == LSK_EPI_RESIDUAL)
-      gemm_f32_kernel<LSK_EPI_RESIDUAL><<<grid, 256, 0, s>>>(a, lda, w, ldw, c, ldc, r, ldr, M, N, K, ffn);
-    else if (epilogue == LSK_EPI_SILU_MUL)
-      gemm_f32_kernel<LSK_EPI_SILU_MUL><<<grid, 256, 0, s>>>(a, lda, w, ldw, c, ldc, r, ldr, M, N, K, ffn);
+    const float* r = epilogue == LSK_EPI_RESIDUAL ? (const float*)R : nullptr;
+    if (epilogue == LSK_EPI_SILU_MUL)
+      launch_f32<true>(s, a, lda, w, ldw, (float*)C, ldc, r, ldr, M, N, K, ffn);
     else
-      gemm_f32_kernel<LSK_EPI_NONE><<<grid, 256, 0, s>>>(a, lda, w, ldw, c, ldc, r, ldr, M, N, K, ffn);
+      launch_f32<false>(s, a, lda, w, ldw, (float*)C, ldc, r, ldr, M, N, K, ffn);
     return lsk_check_launch("lsk_gemm(f32)");
   }
   LSK_REQUIRE(false, LSK_EUNSUPPORTED, "lsk_gemm: dtype %d", dtype);

@@ -148,6 +148,29 @@ def test_gemm_f32(cuda, M, N, K):
     assert torch.allclose(got, F.silu(gg) * uu, rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 9, 64), (2, 40, 320), (4, 33, 1000), (5, 17, 4160), (8, 24, 576), (9, 4100, 70),
+                                   (17, 4097, 520), (31, 4096, 64), (33, 50, 777), (121, 19, 260)])
+def test_gemm_f32_is_bitwise_the_ordered_sums(cuda, M, N, K):
+    """Every tile of the fp32 GEMM (row counts either side of each tile edge, ragged weight rows, whole and partial
+    units of k, strided A) gives bitwise the oracle's lane sums and tree; residual and silu-mul on top of them."""
+    from oracle.ordered import linear, silu_f32
+
+    lsk = _lsk()
+    g = _gen(M * 1000 + K)
+    a, w = torch.randn(M, K + 3, generator=g)[:, 1:K + 1], torch.randn(2 * N, K, generator=g)
+    r = torch.randn(M, N, generator=g)
+    y = linear(a.numpy(), w.numpy())
+    ad = a.to(cuda)
+    ad = torch.nn.functional.pad(ad, (1, 2))[:, 1:K + 1]     # row stride K + 3, first element not 16-byte aligned
+    assert ad.stride(0) == K + 3
+    wd, rd = w.to(cuda), r.to(cuda)
+    assert np.array_equal(lsk.gemm(ad, wd[:N].contiguous()).cpu().numpy(), y[:, :N])
+    got = lsk.gemm(ad, wd[:N].contiguous(), residual=rd, epilogue=lsk.EPI_RESIDUAL)
+    assert np.array_equal(got.cpu().numpy(), r.numpy() + y[:, :N])
+    got = lsk.gemm(ad, wd, epilogue=lsk.EPI_SILU_MUL)
+    assert np.array_equal(got.cpu().numpy(), silu_f32(y[:, :N]) * y[:, N:])
+
+
 # ----------------------------------------------------------------------------- RMSNorm
 
 @pytest.mark.parametrize("dtype", [BF16, F32])
@@ -339,6 +362,23 @@ def test_ragged_attention_f32_matches_brute_force(cuda):
     q, kc, vc, tab, ref = _attn_case(9, F32, 3, 4, 2, 16, 256, [(0, 3, 1), (1, 30, 5), (2, 100, 9)])
     got = _run_attn(lsk, cuda, q, kc, vc, tab, 1 << 30).double()
     assert (got - ref).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(16, 4, 2), (32, 6, 2), (64, 32, 8), (128, 4, 4)])
+def test_ragged_attention_f32_is_bitwise_the_ordered_one(cuda, D, Hq, Hkv):
+    """Chunk edges (positions 0, 31, 32, 63, 64, 127, 128), the cache's last position and items of one to 48 rows:
+    bitwise the oracle's ordered attention."""
+    from oracle.ordered import attend
+
+    lsk = _lsk()
+    blocks = [(0, 0, 1), (1, 30, 3), (2, 60, 9), (3, 126, 25), (4, 191, 1)]
+    q, kc, vc, tab, _ = _attn_case(D, F32, 5, Hq, Hkv, D, 192, blocks)
+    rows = [r for r, _, T in blocks for _ in range(T)]
+    pos = [p + t for _, p, T in blocks for t in range(T)]
+    want = attend(q.numpy(), kc.numpy(), vc.numpy(), rows, pos, Hq // Hkv).reshape(len(rows), Hq * D)
+    for cap in (16, 48):
+        got = _run_attn(lsk, cuda, q, kc, vc, tab, 1 << 30, cap)
+        assert np.array_equal(got.numpy(), want), cap
 
 
 def test_ragged_attention_bf16_is_batch_invariant(cuda):
