@@ -41,9 +41,6 @@ __device__ __forceinline__ float rbf(float f) { return bf2f(f2bf(f)); }
 // operation and the build contracts nothing into FMAs, so a host restatement of the same steps (the fp32
 // oracle's) produces the same bits.  Used by the fp32 attention softmax and by SiLU.
 __device__ __forceinline__ float lsk_exp(float x) {
-  if (x != x) return x;
-  if (x < -86.0f) return 0.0f;
-  if (x > 89.0f) return __builtin_huge_valf();
   const float n = __builtin_rintf(x * 1.4426950216293335f);
   const float r = (x - n * 0.693145751953125f) - n * 1.428606765330187e-06f;
   float p = 0.00019841270113829523f;
@@ -54,7 +51,9 @@ __device__ __forceinline__ float lsk_exp(float x) {
   p = p * r + 0.5f;
   p = p * r + 1.0f;
   p = p * r + 1.0f;
-  return __builtin_ldexpf(p, (int)n);
+  // selects instead of early returns: the lanes of a wave would take both sides anyway
+  const float e = __builtin_ldexpf(p, (int)fminf(fmaxf(n, -200.0f), 200.0f));
+  return x != x ? x : (x < -86.0f ? 0.0f : (x > 89.0f ? __builtin_huge_valf() : e));
 }
 
 // Offset of K cache element (position p, dim d) within one (row, KV head) stripe of S positions x D.
@@ -152,6 +151,7 @@ int lsk_gemm_partial_af(const void* A, const void* W, float* P, int M, int N, in
 // w13 with silu-mul over a fragment-major A; H row-major ([M, ffn]) or, with h_frag, fragment-major (whole
 // 16-token groups) for the w2 launch.
 int lsk_gemm_silu_af(const void* A, const void* W, void* H, int h_frag, int M, int ffn, int K, void* stream);
+bool lsk_gemm_residual_covers(int M, int N, int K, int ks);
 int lsk_ragged_attn_impl(int dtype, const void* q, const void* kcache, const void* vcache, const int32_t* blocks,
                          const int32_t* works, int n_works, const int32_t* groups, int n_groups, int n_parts,
                          const int32_t* recs, int n_rounds, int n_slots, int rows_cap, void* out, int out_frag,

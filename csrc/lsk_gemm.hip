@@ -35,58 +35,8 @@
 #include <type_traits>
 
 #include "lsk_common.h"
+#include "lsk_gemm.h"
 #include "../include/lsk.h"
-
-#define EPI_PARTIAL 3
-#define EPI_ARGMAX 4
-#define EPI_QKV 5
-
-// Fused qkv epilogue (EPI_QKV): the qkv projection's output goes straight to RoPE and the caches instead of through
-// K-slice partials and the RoPE + append kernel.  The weight is packed with its q and k row groups RoPE-paired
-// (lsk_pack_weight_qkv): within each head of D rows (G = D / 16 groups) packed group 2 j holds dims 16 j .. 16 j + 15
-// and packed group 2 j + 1 dims D / 2 + 16 j .. (the rotation partners), so a tile of two (or four) row groups holds
-// whole rotation pairs and one lane owns both values of a pair.  v rows keep their order.
-struct QkvRope {
-  uint16_t* q;            // [N, Hq, D] RoPE-rotated queries
-  uint16_t* kc;           // K cache, fragment-major 32-position blocks (k_cache_offset)
-  uint16_t* vc;           // V cache, transposed 32-position blocks
-  const float* cos_tab;   // [tab_len, D] fp32
-  const float* sin_tab;
-  const int32_t* rows;    // [N] cache row of each token
-  const int32_t* pos;     // [N] position of each token
-  int hq, hkv, d, max_batch, max_seq, tab_len;
-};
-
-// Token m's values x_lo, x_hi of packed row groups G (even) and G + 1, row w16 of each: a RoPE pair for q / k (stored
-// rotated to q or the K cache), two v dims 16 apart otherwise (stored to the V cache), with the RoPE + append
-// kernel's arithmetic (rope_pair) and indexing.
-__device__ __forceinline__ void qkv_rope_store(const QkvRope& qa, int m, int G, int w16, float x_lo, float x_hi) {
-  const int D = qa.d, GH = D >> 4, half = D >> 1;
-  const int row = qa.rows[m], p = qa.pos[m];
-  if (row < 0 || row >= qa.max_batch || p < 0 || p >= qa.max_seq || p >= qa.tab_len) return;  // host validates too
-  const int kg = (qa.hq + qa.hkv) * GH;
-  if (G < kg) {
-    const int h = G / GH, d1 = 16 * ((G - h * GH) >> 1) + w16;
-    float o1, o2;
-    rope_pair<uint16_t>(x_lo, x_hi, qa.cos_tab + (long)p * D, qa.sin_tab + (long)p * D, d1, half, o1, o2);
-    if (h < qa.hq) {
-      uint16_t* dst = qa.q + ((long)m * qa.hq + h) * D;
-      dst[d1] = f2bf(o1);
-      dst[d1 + half] = f2bf(o2);
-    } else {
-      uint16_t* dst = qa.kc + ((long)row * qa.hkv + (h - qa.hq)) * (long)qa.max_seq * D;
-      dst[k_cache_offset<uint16_t>(p, d1, D)] = f2bf(o1);
-      dst[k_cache_offset<uint16_t>(p, d1 + half, D)] = f2bf(o2);
-    }
-  } else {
-    const int gv = G - kg, h = gv / GH, d1 = 16 * (gv - h * GH) + w16;
-    uint16_t* dst = qa.vc + ((long)row * qa.hkv + h) * (long)D * qa.max_seq + (long)(p >> 5) * 32 * D + (p & 31);
-    dst[(long)d1 * 32] = f2bf(x_lo);
-    dst[(long)(d1 + 16) * 32] = f2bf(x_hi);
-  }
-}
-
-__device__ __forceinline__ float silu_f(float x) { return x / (1.0f + lsk_exp(-x)); }
 
 // One lane's 16 bytes of a weight fragment, non-temporal (streamed once per launch).
 __device__ __forceinline__ lsk_bf16x8 ld_w(const uint16_t* p) {
@@ -984,7 +934,7 @@ struct WideCfg {
   int ns, m_blocks, tbg, msw;
 };
 
-static WideCfg wide_config(int epi, int M, int N, int ks) {
+static WideCfg wide_config(int epi, int M, int N, int ks, double* cost_out = nullptr) {
   const bool silu = epi == LSK_EPI_SILU_MUL;
   const int gtot = (M + 15) / 16;
   WideCfg best{0, 0, 0, 0};
@@ -1011,6 +961,7 @@ static WideCfg wide_config(int epi, int M, int N, int ks) {
       }
     }
   }
+  if (cost_out) *cost_out = best_cost;
   return best;
 }
 
@@ -1046,6 +997,42 @@ static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_o
   const int narrow = (epi == EPI_QKV || epi == LSK_EPI_SILU_MUL) ? 32 : 64;
   if ((long)(N / narrow) * ((gtot + 23) / 24) * ks < 128) return none;
   return wide_config(epi, M, N, ks);
+}
+
+// The many-token tier's configuration where it takes a fragment-major launch (mg == 0: it does not).  From
+// LSK_DEEP_ALWAYS_TOKENS rows on it always does (faster or within 5 % at every projection of the 1B, 7B and 8B shapes);
+// from LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's (its cost in us: fitted to the same
+// measurements, within 25 %): qkv of the 8B shape at 256 / 352 / 512 rows 39 / 39 / 40 us against the wide tier's 38 /
+// 47 / 57, w13 at 352 / 448 rows 124 / 136 against 113 / 163.
+static DeepCfg deep_plan(int epi, int M, int N, int K, int ks) {
+  const DeepCfg none{0, 0, 0, 0.0};
+  const DeepCfg d = lsk_deep_plan(epi, M, N, K, ks);
+  if (d.mg == 0 || M >= LSK_DEEP_ALWAYS_TOKENS) return d;
+  double cost = 0.0;
+  if (wide_plan(epi, M, N, K, ks, true, true).ns == 0) return none;  // (few weight tiles: the decode tier)
+  wide_config(epi, M, N, ks, &cost);
+  cost *= (double)(K / ks) / 4096.0;
+  double us;
+  if (epi == LSK_EPI_SILU_MUL) us = 15.8 * cost + 9.0;
+  else if (epi == EPI_PARTIAL) us = 8.5 * cost + 4.5 + 1.7 * ks * (double)M * N * 4.0 / 4.5e6;
+  else us = 11.1 * cost + 4.5;
+  // the partials' and the head's estimates scatter more
+  return d.us < (epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9) * us ? d : none;
+}
+
+extern "C" int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, int* cfg) {
+  LSK_REQUIRE(cfg != nullptr, LSK_EARG, "lsk_gemm_deep_config: null pointer");
+  LSK_REQUIRE(epilogue >= LSK_EPI_NONE && epilogue <= EPI_QKV, LSK_EARG, "lsk_gemm_deep_config: epilogue %d", epilogue);
+  DeepCfg c{0, 0, 0, 0.0};
+  if (epilogue == LSK_EPI_RESIDUAL) {
+    if (lsk_gemm_residual_covers(M, N, K, ks)) c = lsk_deep_plan(epilogue, M, N, K, ks);
+  } else if (epilogue != LSK_EPI_NONE) {
+    c = deep_plan(epilogue, M, N, K, ks);
+  }
+  cfg[0] = c.mg;
+  cfg[1] = c.m_blocks;
+  cfg[2] = c.split;
+  return 0;
 }
 
 extern "C" int lsk_gemm_wide_config(int epilogue, int M, int N, int K, int ks, int af, int* cfg) {
@@ -1213,6 +1200,12 @@ extern "C" int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw
 // with the same tiles (so the same sums).  c_nks > 0 (silu-mul): C fragment-major too.
 static void gemm_af(int epi, hipStream_t s, const void* A, const void* W, void* C, long ldc, int c_nks, float* P,
                     float* av, int* ai, int M, int N, int K, int ffn, int ks) {
+  const DeepCfg deep = deep_plan(epi, M, N, K, ks);
+  if (deep.mg > 0) {
+    lsk_gemm_deep(deep, epi, s, (const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, ldc, c_nks, nullptr, P, av, ai, M, N,
+                  K, ffn, ks, QkvRope{});
+    return;
+  }
   const int mw = launch_wide(epi, s, (const uint16_t*)A, 0, (const uint16_t*)W, (uint16_t*)C, ldc, nullptr, 0, P, av,
                              ai, M, N, K, ffn, ks, true, c_nks);
   if (mw == M) return;
@@ -1240,6 +1233,26 @@ int lsk_gemm_silu_af(const void* A, const void* W, void* H, int h_frag, int M, i
   gemm_af(LSK_EPI_SILU_MUL, (hipStream_t)stream, A, W, H, ffn, h_frag ? ffn / 32 : 0, nullptr, nullptr, nullptr, M,
           ffn, K, ffn, 1);
   return lsk_check_launch("lsk_gemm_silu_af");
+}
+
+// Whether the o / w2 projection of M rows sums its K slices in the GEMM (lsk_gemm_residual_frag) instead of leaving
+// partials for the next add + RMSNorm.
+bool lsk_gemm_residual_covers(int M, int N, int K, int ks) {
+  return M >= LSK_DEEP_ALWAYS_TOKENS && lsk_deep_sums(M, N, K, ks);
+}
+
+extern "C" int lsk_gemm_residual_frag(const void* A, const void* W, const void* R, void* C, int M, int N, int K, int ks,
+                                      void* stream) {
+  LSK_REQUIRE(A && W && R && C, LSK_EARG, "lsk_gemm_residual_frag: null pointer");
+  LSK_REQUIRE(M >= 0 && N > 0 && N % 16 == 0 && K > 0 && ks >= 1 && K % ks == 0 && (K / ks) % 32 == 0, LSK_ESHAPE,
+              "lsk_gemm_residual_frag: bad shape M=%d N=%d K=%d ks=%d", M, N, K, ks);
+  if (M == 0) return 0;
+  const DeepCfg deep = lsk_deep_plan(LSK_EPI_RESIDUAL, M, N, K, ks);
+  LSK_REQUIRE(deep.mg > 0, LSK_EUNSUPPORTED, "lsk_gemm_residual_frag: M=%d N=%d K=%d ks=%d is not a many-token launch", M,
+              N, K, ks);
+  lsk_gemm_deep(deep, LSK_EPI_RESIDUAL, (hipStream_t)stream, (const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, N, 0,
+                (const uint16_t*)R, nullptr, nullptr, nullptr, M, N, K, 0, ks, QkvRope{});
+  return lsk_check_launch("lsk_gemm_residual_frag");
 }
 
 extern "C" int lsk_gemm_partial_frag(const void* A, const void* W, float* P, int M, int N, int K, int ks, void* stream) {
@@ -1394,6 +1407,12 @@ extern "C" int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_head
   const QkvRope qa{(uint16_t*)q_out, (uint16_t*)kcache, (uint16_t*)vcache, cos_tab, sin_tab, rows, pos, n_heads,
                    n_kv_heads, head_dim, max_batch, max_seq, tab_len};
   hipStream_t s = (hipStream_t)stream;
+  const DeepCfg deep = deep_plan(EPI_QKV, M, N, K, 1);
+  if (deep.mg > 0) {
+    lsk_gemm_deep(deep, EPI_QKV, s, (const uint16_t*)A, (const uint16_t*)W, nullptr, 0, 0, nullptr, nullptr, nullptr,
+                  nullptr, M, N, K, 0, 1, qa);
+    return lsk_check_launch("lsk_gemm_qkv_rope(deep)");
+  }
   const int mw = launch_wide(EPI_QKV, s, (const uint16_t*)A, 0, (const uint16_t*)W, nullptr, 0, nullptr, 0, nullptr,
                              nullptr, nullptr, M, N, K, 0, 1, true, 0, qa);
   if (mw < M) {

@@ -250,6 +250,10 @@ extern "C" int lsk_forward_layers(long handle, const void* x_in, void* x_out, in
     const int af = m->dim % 32 == 0;
     const int af_o = qd % 32 == 0;
     const int af_h = N > LSK_AF_MAX_TOKENS && m->dim % 32 == 0 && m->ffn % 64 == 0;
+    // many tokens: the o / w2 GEMM sums its K slices itself and writes the residual stream, so no partials travel
+    // through memory and the next norm is a plain one
+    const bool res_o = af_o && lsk_gemm_residual_covers(N, m->dim, qd, m->ks_o);
+    const bool res_2 = af_h && lsk_gemm_residual_covers(N, m->dim, m->ffn, m->ks_w2);
     const double norm_bytes_b = es_d * (2.0 * Nd * dimd + dimd);
     auto pbytes = [&](int ks, double width) { return 4.0 * ks * Nd * width; };
 #define LSK_PROF2(cls, b, f, call)                               \
@@ -264,9 +268,14 @@ extern "C" int lsk_forward_layers(long handle, const void* x_in, void* x_out, in
                   lsk_add_rmsnorm_impl(m->dtype, x_in, m->dim, nullptr, 0, m->attn_norm[i], m->eps, nullptr, 0, xn,
                                        m->dim, af, N, m->dim, stream));
       } else {
-        LSK_PROF2(LSK_PROF_NORM, norm_bytes_b + es_d * Nd * dimd + pbytes(m->ks_w2, dimd), 4.0 * Nd * dimd,
-                  lsk_add_rmsnorm_impl(m->dtype, x_out, m->dim, P, m->ks_w2, m->attn_norm[i], m->eps, x_out, m->dim,
-                                       xn, m->dim, af, N, m->dim, stream));
+        if (res_2)
+          LSK_PROF2(LSK_PROF_NORM, norm_bytes_b, 4.0 * Nd * dimd,
+                    lsk_add_rmsnorm_impl(m->dtype, x_out, m->dim, nullptr, 0, m->attn_norm[i], m->eps, nullptr, 0, xn,
+                                         m->dim, af, N, m->dim, stream));
+        else
+          LSK_PROF2(LSK_PROF_NORM, norm_bytes_b + es_d * Nd * dimd + pbytes(m->ks_w2, dimd), 4.0 * Nd * dimd,
+                    lsk_add_rmsnorm_impl(m->dtype, x_out, m->dim, P, m->ks_w2, m->attn_norm[i], m->eps, x_out, m->dim,
+                                         xn, m->dim, af, N, m->dim, stream));
         if (capture && capture[i - 1]) {
           hipError_t e = hipMemcpyAsync(capture[i - 1], x_out, (size_t)N * m->dim * es, hipMemcpyDeviceToDevice, s);
           if (e != hipSuccess) { lsk_set_error("lsk_forward_layers: capture %s", hipGetErrorString(e)); return (int)e; }
@@ -282,24 +291,37 @@ extern "C" int lsk_forward_layers(long handle, const void* x_in, void* x_out, in
                 lsk_ragged_attn_impl(m->dtype, q, m->kc[i], m->vc[i], blocks, works, n_works, groups, n_groups,
                                      n_parts, recs, n_rounds, n_slots, rows_cap, attn, af_o, m->n_heads,
                                      m->n_kv_heads, m->head_dim, m->max_seq, scale, part, part_bytes, stream));
-      LSK_PROF2(LSK_PROF_GEMM_O, es_d * (dimd * qd + Nd * qd) + pbytes(m->ks_o, dimd), 2.0 * Nd * qd * dimd,
-                af_o ? lsk_gemm_partial_af(attn, m->wo[i], P, N, m->dim, qd, m->ks_o, stream)
-                     : lsk_gemm_partial(attn, qd, m->wo[i], qd, P, N, m->dim, qd, m->ks_o, stream));
       const void* xi = (i == start) ? x_in : x_out;
-      LSK_PROF2(LSK_PROF_NORM, norm_bytes_b + es_d * Nd * dimd + pbytes(m->ks_o, dimd), 4.0 * Nd * dimd,
-                lsk_add_rmsnorm_impl(m->dtype, xi, m->dim, P, m->ks_o, m->ffn_norm[i], m->eps, x_out, m->dim, xn,
-                                     m->dim, af_h, N, m->dim, stream));
+      if (res_o) {
+        LSK_PROF2(LSK_PROF_GEMM_O, es_d * (dimd * qd + Nd * qd + 2.0 * Nd * dimd), 2.0 * Nd * qd * dimd,
+                  lsk_gemm_residual_frag(attn, m->wo[i], xi, x_out, N, m->dim, qd, m->ks_o, stream));
+        LSK_PROF2(LSK_PROF_NORM, norm_bytes_b, 4.0 * Nd * dimd,
+                  lsk_add_rmsnorm_impl(m->dtype, x_out, m->dim, nullptr, 0, m->ffn_norm[i], m->eps, nullptr, 0, xn,
+                                       m->dim, af_h, N, m->dim, stream));
+      } else {
+        LSK_PROF2(LSK_PROF_GEMM_O, es_d * (dimd * qd + Nd * qd) + pbytes(m->ks_o, dimd), 2.0 * Nd * qd * dimd,
+                  af_o ? lsk_gemm_partial_af(attn, m->wo[i], P, N, m->dim, qd, m->ks_o, stream)
+                       : lsk_gemm_partial(attn, qd, m->wo[i], qd, P, N, m->dim, qd, m->ks_o, stream));
+        LSK_PROF2(LSK_PROF_NORM, norm_bytes_b + es_d * Nd * dimd + pbytes(m->ks_o, dimd), 4.0 * Nd * dimd,
+                  lsk_add_rmsnorm_impl(m->dtype, xi, m->dim, P, m->ks_o, m->ffn_norm[i], m->eps, x_out, m->dim, xn,
+                                       m->dim, af_h, N, m->dim, stream));
+      }
       LSK_PROF2(LSK_PROF_GEMM_W13, es_d * (2.0 * ffd * dimd + Nd * dimd + Nd * ffd), 4.0 * Nd * dimd * ffd,
                 af_h ? lsk_gemm_silu_af(xn, m->w13[i], h, 1, N, m->ffn, m->dim, stream)
                      : lsk_gemm(m->dtype, xn, m->dim, m->w13[i], m->dim, h, m->ffn, nullptr, 0, N, m->ffn, m->dim,
                                 LSK_EPI_SILU_MUL, m->ffn, stream));
-      LSK_PROF2(LSK_PROF_GEMM_W2, es_d * (dimd * ffd + Nd * ffd) + pbytes(m->ks_w2, dimd), 2.0 * Nd * ffd * dimd,
-                af_h ? lsk_gemm_partial_af(h, m->w2[i], P, N, m->dim, m->ffn, m->ks_w2, stream)
-                     : lsk_gemm_partial(h, m->ffn, m->w2[i], m->ffn, P, N, m->dim, m->ffn, m->ks_w2, stream));
+      if (res_2)
+        LSK_PROF2(LSK_PROF_GEMM_W2, es_d * (dimd * ffd + Nd * ffd + 2.0 * Nd * dimd), 2.0 * Nd * ffd * dimd,
+                  lsk_gemm_residual_frag(h, m->w2[i], x_out, x_out, N, m->dim, m->ffn, m->ks_w2, stream));
+      else
+        LSK_PROF2(LSK_PROF_GEMM_W2, es_d * (dimd * ffd + Nd * ffd) + pbytes(m->ks_w2, dimd), 2.0 * Nd * ffd * dimd,
+                  af_h ? lsk_gemm_partial_af(h, m->w2[i], P, N, m->dim, m->ffn, m->ks_w2, stream)
+                       : lsk_gemm_partial(h, m->ffn, m->w2[i], m->ffn, P, N, m->dim, m->ffn, m->ks_w2, stream));
     }
-    LSK_PROF2(LSK_PROF_NORM, 2.0 * es_d * Nd * dimd + pbytes(m->ks_w2, dimd), Nd * dimd,
-              lsk_add_rmsnorm(m->dtype, x_out, m->dim, P, m->ks_w2, nullptr, m->eps, x_out, m->dim, nullptr, 0, N,
-                              m->dim, stream));
+    if (!res_2)
+      LSK_PROF2(LSK_PROF_NORM, 2.0 * es_d * Nd * dimd + pbytes(m->ks_w2, dimd), Nd * dimd,
+                lsk_add_rmsnorm(m->dtype, x_out, m->dim, P, m->ks_w2, nullptr, m->eps, x_out, m->dim, nullptr, 0, N,
+                                m->dim, stream));
     if (capture && capture[end - 1]) {
       hipError_t e = hipMemcpyAsync(capture[end - 1], x_out, (size_t)N * m->dim * es, hipMemcpyDeviceToDevice, s);
       if (e != hipSuccess) { lsk_set_error("lsk_forward_layers: capture %s", hipGetErrorString(e)); return (int)e; }

@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define LSK_ABI_VERSION 11
+#define LSK_ABI_VERSION 12
 
 #define LSK_EPI_NONE 0     /* C = rnd(A W^T)                                   */
 #define LSK_EPI_RESIDUAL 1 /* C = rnd(R + rnd(A W^T))                          */
@@ -147,6 +147,10 @@ int lsk_gemm(int dtype, const void* A, long lda, const void* W, long ldw, void* 
  * reduction order never depends on the token count M; each launch picks its own tile width from M. */
 int lsk_gemm_plan(int N, int K, int* ns_out, int* ks_out);
 
+/* The many-token tier's configuration of a fragment-major launch (epilogue as lsk_gemm_wide_config's; LSK_EPI_RESIDUAL:
+ * lsk_gemm_residual_frag where the layer runner uses it): cfg = {16-token groups per workgroup (0: another tier runs
+ * the launch), token blocks, workgroups sharing a tile's K slices}.  Host only. */
+int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, int* cfg);
 /* Configuration the wide-M tier (the bf16 GEMM path above 64 tokens) picks for a launch: cfg[4] = {ns (16-row
  * groups per tile; 0: the tier does not take the launch), blocks, 16-token groups per block, groups per wave}.
  * epilogue: LSK_EPI_*, or 3 = K-slice partials (lsk_gemm_partial), 4 = LM head + argmax, 5 = fused qkv + RoPE +
@@ -169,6 +173,11 @@ int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw, float* P,
  * launches, exported so that measurements replay exactly those. */
 int lsk_gemm_partial_frag(const void* A, const void* W, float* P, int M, int N, int K, int ks, void* stream);
 int lsk_gemm_silu_frag(const void* A, const void* W, void* H, int h_frag, int M, int ffn, int K, void* stream);
+/* The o / w2 projection of a many-token segment: C = rnd(R + rnd(sum_s P[s])) over lsk_gemm_partial_frag's K-slice
+ * partials P, in slice order, without storing them (bitwise lsk_gemm_partial_frag followed by lsk_add_rmsnorm's x_out).
+ * R and C are [M, N] rows and may be the same buffer.  LSK_EUNSUPPORTED for a shape outside the many-token tier. */
+int lsk_gemm_residual_frag(const void* A, const void* W, const void* R, void* C, int M, int N, int K, int ks,
+                           void* stream);
 
 /* LM head + greedy pick (W packed, ldw == K): out[dst_idx ? dst_idx[m] : m] = argmax_n rnd(A[m] . W[n]) (first index on ties),
  * optionally also storing the bf16 logits [M, ldl].  workspace >= lsk_head_workspace_bytes(M, N).

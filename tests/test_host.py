@@ -1052,3 +1052,28 @@ def test_empty_inputs_return_before_any_launch():
     assert lib.lsk_kv_rollback(P, P, P, 0, None) == 0
     assert lib.lsk_shift_segment_positions(P, 4, 1, 1, 0, 1, 4, P, P, P, 0, None) == 0
     assert lib.lsk_gemm_qkv_rope(P, P, 0, 32, 8, 128, 4096, P, P, P, P, P, 64, P, P, 2, 64, None) == 0
+
+
+def test_deep_config_covers_every_tile_and_every_token_block():
+    """The many-token tier's plan over the presets' projections: every group count and both slice treatments occur, the
+    blocks hold all token groups, and shapes it cannot take (ragged rows, short slices, few tokens) are left alone."""
+    from thesis_amd import _lsk as lsk
+
+    seen = set()
+    for N, K, ks, epi in ((6144, 4096, 1, 5), (4096, 4096, 4, 3), (14336, 4096, 1, 2), (4096, 14336, 4, 3),
+                          (3072, 2048, 1, 5), (2048, 2048, 8, 3), (8192, 2048, 1, 2), (2048, 8192, 8, 3),
+                          (4096, 4096, 4, 1), (4096, 14336, 4, 1), (2048, 2048, 8, 1)):
+        for M in (65, 255, 256, 352, 512, 767, 768, 1024, 1517, 2048, 4001):
+            mg, mb, split = lsk.gemm_deep_config(epi, M, N, K, ks)
+            if M < 256:
+                assert mg == 0
+            if mg:
+                seen.add((mg, split > 1, epi))
+                groups = (M + 15) // 16
+                assert mg in (4, 6, 8) and (mb - 1) * mg < groups <= mb * mg and ks % split == 0
+            elif epi != 1:
+                assert M < 768
+    assert {m for m, _, _ in seen} == {4, 6, 8} and any(sp for _, sp, _ in seen) and any(e == 1 for _, _, e in seen)
+    assert lsk.gemm_deep_config(3, 1024, 4096 + 16, 4096, 4)[0] == 0
+    assert lsk.gemm_deep_config(3, 1024, 4096, 4096 + 64, 1)[0] == 0
+    assert lsk.gemm_deep_config(2, 1024, 64, 4096, 1)[0] == 0

@@ -753,6 +753,47 @@ def test_fragment_major_gemms_are_bitwise_the_row_major_ones(cuda, M):
     assert torch.equal(back.unpack()[:M], h_row)
 
 
+@pytest.mark.parametrize("M,N,K,ks", [(256, 8192, 1024, 1), (768, 256, 128, 1), (769, 512, 512, 4), (783, 2048, 2048, 8),
+                                      (800, 4096, 1024, 4), (1025, 1024, 1536, 2), (1100, 8192, 512, 1),
+                                      (2000, 4096, 768, 1), (2049, 2048, 1280, 2)])
+def test_many_token_gemms_are_bitwise_the_decode_kernel(cuda, M, N, K, ks):
+    """The many-token tier (4, 6 and 8 token groups per workgroup, slices split over workgroups or summed in one, chunk
+    classes with and without chunks, ragged last groups): partials, silu-mul (row- and fragment-major), residual and
+    the head's logits and ids are bitwise those of 64-row (decode tier) launches over the same rows."""
+    lsk = _lsk()
+    g = _gen(M + N + K)
+    m16 = lsk.frag_rows(M)
+    a = torch.randn(m16, K, generator=g).to(BF16).to(cuda)
+    af = lsk.PackedWeight(a).data
+    w = lsk.PackedWeight((torch.randn(N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    parts = [(lo, min(lo + 64, M)) for lo in range(0, M, 64)]
+    want = torch.cat([lsk.gemm_partial(a[lo:hi].contiguous(), w, ks) for lo, hi in parts], dim=1)
+    assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, M, N, K, ks)[0] > 0 or M < 768
+    assert torch.equal(lsk.gemm_partial_frag(af, M, w, ks), want)
+    if lsk.gemm_deep_config(lsk.EPI_RESIDUAL, M, N, K, ks)[0]:
+        r = torch.randn(M, N, generator=g).to(BF16).to(cuda)
+        x = torch.empty_like(r)
+        lsk.add_rmsnorm(r, want, None, 1e-5, x_out=x)
+        assert torch.equal(lsk.gemm_residual_frag(af, M, w, ks, r), x)
+        assert torch.equal(lsk.gemm_residual_frag(af, M, w, ks, r, out=r), x)      # in place
+    w13 = lsk.PackedWeight((torch.randn(2 * N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    want = torch.cat([lsk.gemm(a[lo:hi].contiguous(), w13, epilogue=lsk.EPI_SILU_MUL) for lo, hi in parts])
+    h = torch.empty(M, N, dtype=BF16, device=cuda)
+    assert torch.equal(lsk.gemm_silu_frag(af, M, w13, h, False), want)
+    h = torch.empty(m16 * N, dtype=BF16, device=cuda)
+    lsk.gemm_silu_frag(af, M, w13, h, True)
+    back = lsk.PackedWeight.__new__(lsk.PackedWeight)
+    back.shape, back.dtype, back.device, back.data = (m16, N), BF16, h.device, h
+    assert torch.equal(back.unpack()[:M], want)
+    nw = torch.ones(K, dtype=BF16, device=cuda)
+    ids, lo_ = torch.empty(M, dtype=torch.long, device=cuda), torch.empty(M, N, dtype=BF16, device=cuda)
+    lsk.head_norm_argmax(a[:M].contiguous(), nw, 1e-5, w, ids, logits=lo_)
+    for lo, hi in parts:
+        i1, l1 = torch.empty(hi - lo, dtype=torch.long, device=cuda), torch.empty(hi - lo, N, dtype=BF16, device=cuda)
+        lsk.head_norm_argmax(a[lo:hi].contiguous(), nw, 1e-5, w, i1, logits=l1)
+        assert torch.equal(ids[lo:hi], i1) and torch.equal(lo_[lo:hi], l1)
+
+
 @pytest.mark.parametrize("split", [4096, 128])
 def test_shifted_segment_metadata_equals_a_plan_at_the_actual_positions(cuda, split):
     """A decode segment planned at its verifiers' upper-bound positions (all drafts accepted) and moved back on the

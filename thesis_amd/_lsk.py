@@ -22,7 +22,7 @@ EPI_NONE, EPI_RESIDUAL, EPI_SILU_MUL = 0, 1, 2
 EPI_PARTIAL, EPI_ARGMAX, EPI_QKV_ROPE = 3, 4, 5   # launch kinds known to lsk_gemm_wide_config
 ATTN_SPLIT = 8192         # LSK_ATTN_SPLIT
 ATTN_ROWS = 48            # query rows per attention work item (csrc/lsk_attention.hip ATTN_ROWS)
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 # name -> (restype, argtypes)
 _P, _I, _L, _F, _Z = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_size_t
@@ -50,6 +50,7 @@ _SIGS = {
     "lsk_gemm": (_I, [_I, _P, _L, _P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P]),
     "lsk_gemm_plan": (_I, [_I, _I, _P, _P]),
     "lsk_gemm_wide_config": (_I, [_I, _I, _I, _I, _I, _I, _P]),
+    "lsk_gemm_deep_config": (_I, [_I, _I, _I, _I, _I, _P]),
     "lsk_gemm_partial": (_I, [_P, _L, _P, _L, _P, _I, _I, _I, _I, _P]),
     "lsk_head_workspace_bytes": (_Z, [_I, _I]),
     "lsk_head_argmax": (_I, [_I, _P, _L, _P, _L, _I, _I, _I, _P, _L, _P, _P, _P, _Z, _P]),
@@ -69,6 +70,7 @@ _SIGS = {
     "lsk_segment_workspace_bytes": (_Z, [_L, _I, _I]),
     "lsk_gemm_partial_frag": (_I, [_P, _P, _P, _I, _I, _I, _I, _P]),
     "lsk_gemm_silu_frag": (_I, [_P, _P, _P, _I, _I, _I, _I, _P]),
+    "lsk_gemm_residual_frag": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lsk_forward_layers": (_I, [_L, _P, _P, _I, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _P, _Z, _P,
                                 ctypes.c_double, ctypes.c_double, _P]),
     "lsk_prof_enable": (_I, [_I]),
@@ -611,6 +613,13 @@ def gemm_wide_config(epilogue: int, M: int, N: int, K: int, ks: int = 1, af: boo
     return tuple(cfg)
 
 
+def gemm_deep_config(epilogue: int, M: int, N: int, K: int, ks: int = 1) -> tuple:
+    """(groups, token blocks, split) of a fragment-major launch in the many-token tier; groups 0: another tier."""
+    cfg = (ctypes.c_int * 3)()
+    _check(load().lsk_gemm_deep_config(epilogue, M, N, K, ks, cfg), "lsk_gemm_deep_config")
+    return tuple(cfg)
+
+
 def frag_rows(m: int) -> int:
     """Rows a fragment-major activation buffer of m tokens holds (whole 16-token groups)."""
     return (m + 15) // 16 * 16
@@ -629,6 +638,25 @@ def gemm_partial_frag(a_frag: torch.Tensor, m: int, w: torch.Tensor, ks: int,
         out = torch.empty(ks, m, N, dtype=torch.float32, device=a_frag.device)
     _check(load().lsk_gemm_partial_frag(_ptr(a_frag), _ptr(w), _ptr(out), m, N, K, ks, _stream()),
            "lsk_gemm_partial_frag")
+    return out
+
+
+def gemm_residual_frag(a_frag: torch.Tensor, m: int, w: torch.Tensor, ks: int, residual: torch.Tensor,
+                       out: torch.Tensor | None = None) -> torch.Tensor:
+    """residual + the product of a many-token segment (lsk_gemm_residual_frag): a_frag as gemm_partial_frag's, residual
+    and out [m, N] bf16 rows (out may be residual); the K slices are summed in slice order in the launch."""
+    _dev(a_frag, w, residual, out)
+    _check_weight(a_frag, w)
+    N, K = w.shape
+    if a_frag.dtype != torch.bfloat16 or a_frag.numel() < frag_rows(m) * K or not a_frag.is_contiguous():
+        raise LskError("gemm_residual_frag: a contiguous bf16 buffer of frag_rows(m) x K elements is needed")
+    if out is None:
+        out = torch.empty(m, N, dtype=torch.bfloat16, device=a_frag.device)
+    for t in (residual, out):
+        if t.shape != (m, N) or t.dtype != torch.bfloat16 or not t.is_contiguous():
+            raise LskError("gemm_residual_frag: residual and out must be contiguous [m, N] bf16 tensors")
+    _check(load().lsk_gemm_residual_frag(_ptr(a_frag), _ptr(w), _ptr(residual), _ptr(out), m, N, K, ks, _stream()),
+           "lsk_gemm_residual_frag")
     return out
 
 

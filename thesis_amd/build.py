@@ -11,7 +11,7 @@ import sys
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parents[1]
-SOURCES = ["lsk_elementwise.hip", "lsk_attention.hip", "lsk_gemm.hip", "lsk_runtime.hip"]
+SOURCES = ["lsk_elementwise.hip", "lsk_attention.hip", "lsk_gemm.hip", "lsk_gemm_deep.hip", "lsk_runtime.hip"]
 OUT = ROOT / "thesis_amd" / "_lib" / "liblsk.so"
 
 FLAGS = [
