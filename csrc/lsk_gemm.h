@@ -55,7 +55,7 @@ __device__ __forceinline__ void qkv_rope_store(const QkvRope& qa, int m, int G, 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + lsk_exp(-x)); }
 
 #define LSK_DEEP_MIN_TOKENS 256     // below: the wide tier
-#define LSK_DEEP_ALWAYS_TOKENS 768  // from here on: the many-token tier whatever the estimates
+#define LSK_DEEP_ALWAYS_TOKENS 900  // from here on: the many-token tier whatever the estimates
 // Many-token tier (lsk_gemm_deep.hip) over a fragment-major A: whether it takes a launch, and the launch.  Same sums as
 // the other tiers.
 struct DeepCfg {

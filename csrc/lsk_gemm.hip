@@ -1002,19 +1002,20 @@ static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_o
 // The many-token tier's configuration where it takes a fragment-major launch (mg == 0: it does not).  From
 // LSK_DEEP_ALWAYS_TOKENS rows on it always does (faster or within 5 % at every projection of the 1B, 7B and 8B shapes);
 // from LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's (its cost in us: fitted to the same
-// measurements, within 25 %): qkv of the 8B shape at 256 / 352 / 512 rows 39 / 39 / 40 us against the wide tier's 38 /
-// 47 / 57, w13 at 352 / 448 rows 124 / 136 against 113 / 163.
+// measurements, within 25 %).  Cold weights, 8B shape at 288 / 512 rows: qkv 48 / 54 us against the wide tier's 46 / 59,
+// w13 109 / 143 against 105 / 179, w2 63 / 67 against 51 / 87.
 static DeepCfg deep_plan(int epi, int M, int N, int K, int ks) {
   const DeepCfg none{0, 0, 0, 0.0};
   const DeepCfg d = lsk_deep_plan(epi, M, N, K, ks);
   if (d.mg == 0 || M >= LSK_DEEP_ALWAYS_TOKENS) return d;
   double cost = 0.0;
   if (wide_plan(epi, M, N, K, ks, true, true).ns == 0) return none;  // (few weight tiles: the decode tier)
+  if (epi == EPI_PARTIAL && K / ks < 512) return none;               // a class per chunk: folds and stores dominate
   wide_config(epi, M, N, ks, &cost);
   cost *= (double)(K / ks) / 4096.0;
   double us;
   if (epi == LSK_EPI_SILU_MUL) us = 15.8 * cost + 9.0;
-  else if (epi == EPI_PARTIAL) us = 8.5 * cost + 4.5 + 1.7 * ks * (double)M * N * 4.0 / 4.5e6;
+  else if (epi == EPI_PARTIAL) us = 7.4 * cost + 4.5 + 2.0 * ks * (double)M * N * 4.0 / 4.5e6;
   else us = 11.1 * cost + 4.5;
   // the partials' and the head's estimates scatter more
   return d.us < (epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9) * us ? d : none;

@@ -1063,7 +1063,7 @@ def test_deep_config_covers_every_tile_and_every_token_block():
     for N, K, ks, epi in ((6144, 4096, 1, 5), (4096, 4096, 4, 3), (14336, 4096, 1, 2), (4096, 14336, 4, 3),
                           (3072, 2048, 1, 5), (2048, 2048, 8, 3), (8192, 2048, 1, 2), (2048, 8192, 8, 3),
                           (4096, 4096, 4, 1), (4096, 14336, 4, 1), (2048, 2048, 8, 1)):
-        for M in (65, 255, 256, 352, 512, 767, 768, 1024, 1517, 2048, 4001):
+        for M in (65, 255, 256, 352, 512, 899, 900, 1024, 1517, 2048, 4001):
             mg, mb, split = lsk.gemm_deep_config(epi, M, N, K, ks)
             if M < 256:
                 assert mg == 0
@@ -1072,7 +1072,7 @@ def test_deep_config_covers_every_tile_and_every_token_block():
                 groups = (M + 15) // 16
                 assert mg in (4, 6, 8) and (mb - 1) * mg < groups <= mb * mg and ks % split == 0
             elif epi != 1:
-                assert M < 768
+                assert M < 900
     assert {m for m, _, _ in seen} == {4, 6, 8} and any(sp for _, sp, _ in seen) and any(e == 1 for _, _, e in seen)
     assert lsk.gemm_deep_config(3, 1024, 4096 + 16, 4096, 4)[0] == 0
     assert lsk.gemm_deep_config(3, 1024, 4096, 4096 + 64, 1)[0] == 0
