@@ -838,10 +838,19 @@ static int ms_for(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 48 ? 3 : 4)
 // third of the CUs idle (fewer than 160 workgroups: the 1B MLP's 128) runs 32-row tiles instead.  Measured on
 // MI355X (back-to-back launches, cold weights): 1B w13 -12 % at 8 tokens to -26 % at 64; the 7B MLP (172
 // workgroups) ran 9-13 % slower with 32-row tiles, so it keeps 64.
+// Up to 16 tokens the activations are one fragment per k-step whatever the tile, and more, smaller workgroups stream
+// the weights better (cold weights): silu-mul with 16 + 16 rows at 8 tokens 12.2 / 28.9 / 38.2 us for the 1B / 7B / 8B
+// shapes against 14.9 / 33.1 / 40.8 with 32- or 64-row tiles (16 tokens: 12.8 / 31.2 / 40.6 against 14.9 / 33.9 / 40.7; at
+// 24 the wider tiles win); partials with 32 rows at 8 tokens 19.3 us for w2 of the 8B shape (64 rows: 20.0).  A split-K
+// launch of fewer than one 64-row workgroup per CU takes 32-row tiles at every M: w2 of the 7B shape (128) at 8 / 32 / 48
+// tokens 20.4 / 26.8 / 31.2 -> 15.6 / 19.9 / 24.1 us.
 static int tile_ns(int n, int M, int epi, int kslice = 0, int ks = 1, int short_max = 32) {
+  if (epi == LSK_EPI_SILU_MUL && M <= 16) return 1;
   int ns = 4;
   while (ns > 1 && n % (16 * ns) != 0) ns >>= 1;
-  if (ns == 4 && epi == EPI_PARTIAL && M <= short_max && kslice <= 1024 && (long)(n / 64) * ks < 512) ns = 2;
+  if (ns == 4 && epi == EPI_PARTIAL &&
+      (M <= 16 || (long)(n / 64) * ks < 256 || (M <= short_max && kslice <= 1024 && (long)(n / 64) * ks < 512)))
+    ns = 2;
   if (ns == 4 && epi != EPI_PARTIAL && epi != EPI_ARGMAX && n / 64 < 160 && n % 32 == 0) ns = 2;
   return ns;
 }

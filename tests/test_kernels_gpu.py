@@ -753,6 +753,28 @@ def test_fragment_major_gemms_are_bitwise_the_row_major_ones(cuda, M):
     assert torch.equal(back.unpack()[:M], h_row)
 
 
+@pytest.mark.parametrize("ffn,K", [(16, 512), (48, 1024), (4112, 256), (8192, 2048)])
+def test_small_token_tiles_are_bitwise_the_wider_ones(cuda, ffn, K):
+    """Either side of 16 tokens the silu-mul and split-K launches change their tile width (16- and 32-row tiles up to
+    16; widths that are no multiple of 32 included): a row's result is bitwise the same in both, and the silu-mul is
+    within bf16 rounding of the fp32 product."""
+    lsk = _lsk()
+    g = _gen(ffn + K)
+    a = torch.randn(48, K, generator=g).to(BF16).to(cuda)
+    w13 = (torch.randn(2 * ffn, K, generator=g) * 0.05).to(BF16).to(cuda)
+    wp, w = lsk.PackedWeight(w13), lsk.PackedWeight(w13[:ffn].contiguous())
+    ks = 2 if K % 256 == 0 else 1
+    full, part = lsk.gemm(a, wp, epilogue=lsk.EPI_SILU_MUL), lsk.gemm_partial(a, w, ks)
+    gate, up = (a.float() @ w13.float().t()).chunk(2, dim=-1)
+    ref = F.silu(gate) * up
+    # three bf16 roundings (gate, up, the product), 2^-8 relative each, and the fp32 sums
+    assert ((full.float() - ref).abs() <= 4 * 2.0 ** -8 * ref.abs() + 1e-3).all()
+    for m in (1, 8, 15, 16, 17, 32):
+        x = a[:m].contiguous()
+        assert torch.equal(lsk.gemm(x, wp, epilogue=lsk.EPI_SILU_MUL), full[:m]), m
+        assert torch.equal(lsk.gemm_partial(x, w, ks), part[:, :m]), m
+
+
 @pytest.mark.parametrize("M,N,K,ks", [(256, 8192, 1024, 1), (900, 256, 128, 1), (901, 512, 512, 4), (911, 2048, 2048, 8),
                                       (930, 4096, 1024, 4), (1025, 1024, 1536, 2), (1100, 8192, 512, 1),
                                       (2000, 4096, 768, 1), (2049, 2048, 1280, 2)])
