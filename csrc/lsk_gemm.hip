@@ -74,7 +74,10 @@ __global__ __launch_bounds__(256, (gemm_occupancy<NS, MS, EPI, CK>())) void gemm
   constexpr int NT = (EPI == LSK_EPI_SILU_MUL) ? 2 * NS : NS;
   static_assert(!AF || EPI == EPI_PARTIAL || EPI == EPI_ARGMAX || EPI == LSK_EPI_SILU_MUL || EPI == EPI_QKV,
                 "fragment-major A: split-K partial, silu-mul, LM head and the fused qkv");
-  static_assert(EPI != EPI_QKV || (AF && NS % 2 == 0), "fused qkv: fragment-major A, whole rotation pairs per tile");
+  // fused qkv, whole rotation pairs per tile: two or four row groups, or (NS = 1) eight rows of a group and the same eight
+  // of its partner in the next group (tile 2 p + h: rows 8 h .. 8 h + 7 of groups 2 p and 2 p + 1)
+  static_assert(EPI != EPI_QKV || (AF && (NS == 1 || NS % 2 == 0)), "fused qkv: fragment-major A");
+  constexpr bool HALF = EPI == EPI_QKV && NS == 1;
   constexpr int E = NT * MS * 256;  // partial-sum floats per wave
   __shared__ __attribute__((aligned(16))) float red[4 * E];
 
@@ -106,6 +109,8 @@ __global__ __launch_bounds__(256, (gemm_occupancy<NS, MS, EPI, CK>())) void gemm
     const int gmax = (EPI == LSK_EPI_SILU_MUL) ? (t < NS ? ffn / 16 - 1 : 2 * ffn / 16 - 1) : N / 16 - 1;
     gi = gi < gmax ? gi : gmax;  // clamp: padded row groups load a valid group, results discarded
     wrow[t] = W + ((long)gi * nks + (k0 >> 5)) * 512 + 8 * lane;
+    if constexpr (HALF)  // (eight rows of a fragment are 128 contiguous bytes per 8 columns)
+      wrow[t] = W + ((long)((tn & ~1) + (l16 >> 3)) * nks + (k0 >> 5)) * 512 + 8 * (8 * (tn & 1) + (l16 & 7) + 16 * lg);
   }
   const uint16_t* arow[MS];
 #pragma unroll
@@ -237,23 +242,28 @@ __global__ __launch_bounds__(256, (gemm_occupancy<NS, MS, EPI, CK>())) void gemm
     // consecutive threads take consecutive rows (dims) of a token; v tiles (a 32-row tile never straddles the q / k
     // to v boundary): consecutive tokens of a row, so a verify block's positions land side by side in the
     // transposed V block
-    const bool vtile = n0 / 16 >= (qa.hq + qa.hkv) * (qa.d >> 4);
-    for (int o = tid; o < (NS / 2) * TM * 16; o += 256) {
+    const int g_even = HALF ? (tn & ~1) : n0 / 16;
+    const bool vtile = g_even >= (qa.hq + qa.hkv) * (qa.d >> 4);
+    constexpr int PR = HALF ? 8 : 16, NP = HALF ? 1 : NS / 2;  // rows of a pair in the tile, pairs of groups
+    for (int o = tid; o < NP * TM * PR; o += 256) {
       int w16, ml, pp;
       if (vtile) {
         ml = o % TM;
         const int r2 = o / TM;
-        w16 = r2 & 15;
-        pp = r2 >> 4;
+        w16 = r2 % PR;
+        pp = r2 / PR;
       } else {
-        w16 = o & 15;
-        const int r2 = o >> 4;
+        w16 = o % PR;
+        const int r2 = o / PR;
         ml = r2 % TM;
         pp = r2 / TM;
       }
       const int m = m0 + ml;
       if (m >= M) continue;
-      qkv_rope_store(qa, m, n0 / 16 + 2 * pp, w16, rbf(reduced(2 * pp, ml, w16)), rbf(reduced(2 * pp + 1, ml, w16)));
+      if constexpr (HALF)
+        qkv_rope_store(qa, m, g_even, 8 * (tn & 1) + w16, rbf(reduced(0, ml, w16)), rbf(reduced(0, ml, w16 + 8)));
+      else
+        qkv_rope_store(qa, m, g_even + 2 * pp, w16, rbf(reduced(2 * pp, ml, w16)), rbf(reduced(2 * pp + 1, ml, w16)));
     }
   } else if (EPI == LSK_EPI_SILU_MUL && NS >= 2 && N % 8 == 0 && (ldc % 8 == 0 || c_nks > 0)) {
     // 8 outputs per lane, one 16-byte store: a wave covers 16 tokens x 32 columns per pass (lane l: token
@@ -890,7 +900,7 @@ static void launch_bf16_af(int epi, dim3 grid, hipStream_t s, const uint16_t* A,
     gemm_bf16_kernel<NS, MS, EPI_ARGMAX, gemm_unit<NS, MS, EPI_ARGMAX>(), true><<<grid, 256, 0, s>>>(
         A, 0, W, ldw, C, ldc, nullptr, 0, nullptr, av, ai, M, N, K, 0, kslice, nt, mt, m_lo, 0, QkvRope{});
   else if (epi == EPI_QKV) {
-    if constexpr (NS % 2 == 0)
+    if constexpr (NS == 2 || (NS == 1 && MS == 1))
       gemm_bf16_kernel<NS, MS, EPI_QKV, gemm_unit<NS, MS, EPI_QKV>(), true><<<grid, 256, 0, s>>>(
           A, 0, W, ldw, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, M, N, K, 0, kslice, nt, mt, m_lo, 0, qa);
   } else
@@ -1431,8 +1441,11 @@ extern "C" int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_head
     // tokens 11.9 -> 10.0 us on MI355X
     const int mr = M - mw;
     int ms = ms_for(mr);
+    // up to 16 tokens such a weight runs half-width tiles (8 rotation pairs, twice the workgroups): a 1B decode step of one
+    // token 270.5 -> 265.3 us over 6 layers; with 192 tiles or more they are slower (8B shape 11.8 -> 13.7 us a launch)
+    const int ns = N / 32 < 192 && mr <= 16 ? 1 : 2;
     while (ms > 1 && (long)(N / 32) * ((mr + 16 * ms - 1) / (16 * ms)) < 192) --ms;
-    dispatch_bf16(2, ms, EPI_QKV, N / 32, (mr + 16 * ms - 1) / (16 * ms), 1, s, A, 0, W, K, nullptr, 0, nullptr, 0,
+    dispatch_bf16(ns, ms, EPI_QKV, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, 0, W, K, nullptr, 0, nullptr, 0,
                   nullptr, nullptr, nullptr, M, N, K, 0, K, true, mw, 0, qa);
   }
   return lsk_check_launch("lsk_gemm_qkv_rope");

@@ -908,3 +908,10 @@ def test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, heads):
     assert torch.equal(k2.view(torch.int16), k1.view(torch.int16))
     assert torch.equal(v2.view(torch.int16), v1.view(torch.int16))
     assert not torch.equal(k2, k0) and not torch.equal(v2, v0)
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17])
+def test_fused_qkv_half_width_tiles(cuda, M):
+    """Weights of fewer than 192 32-row tiles run half-width tiles (8 rotation pairs each) up to 16 tokens: the same
+    writes as the unfused path on both sides of that line, q, k and v rows alike."""
+    test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, (8, 2, 64))
