@@ -1215,9 +1215,10 @@ extern "C" int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw
   return lsk_check_launch("lsk_gemm_partial");
 }
 
-// Fragment-major A (lsk_frag_off, whole 16-token groups): above 64 rows the wide tier takes its full token blocks
-// and the decode kernel the rest, exactly as lsk_gemm / lsk_gemm_partial / lsk_head_argmax split a row-major A,
-// with the same tiles (so the same sums).  c_nks > 0 (silu-mul): C fragment-major too.
+// Fragment-major A (lsk_frag_off, whole 16-token groups): the many-token tier where it takes the launch; else above 64
+// rows the wide tier takes its full token blocks and the decode kernel the rest, exactly as lsk_gemm / lsk_gemm_partial
+// / lsk_head_argmax split a row-major A, with the same tiles.  The same sums in all three.  c_nks > 0 (silu-mul): C
+// fragment-major too.
 static void gemm_af(int epi, hipStream_t s, const void* A, const void* W, void* C, long ldc, int c_nks, float* P,
                     float* av, int* ai, int M, int N, int K, int ffn, int ks) {
   const DeepCfg deep = deep_plan(epi, M, N, K, ks);

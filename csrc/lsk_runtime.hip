@@ -8,7 +8,8 @@
 //   q, cache[k, v] = rope(q), rope(k), v              lsk_rope_append          (fp32)
 //   q, cache[k, v] = rope / append of xn Wqkv^T       lsk_gemm_qkv_rope        (bf16: one launch)
 //   attn = ragged attention(q, cache)                 lsk_ragged_attn (+ split combine)
-//   x    = x + attn Wo^T                              lsk_gemm RESIDUAL
+//   x    = x + attn Wo^T                              lsk_gemm RESIDUAL        (bf16: split-K partials that the next
+//                                                     norm adds, or lsk_gemm_residual_frag for long segments)
 //   xn   = rmsnorm(x, ffn_norm)                       lsk_rmsnorm
 //   h    = silu(g) * u, [g; u] = xn W13^T             lsk_gemm SILU_MUL
 //   x    = x + h W2^T                                 lsk_gemm RESIDUAL (in place)
