@@ -1001,8 +1001,12 @@ static void launch_wide_kernel(dim3 grid, hipStream_t s, bool af, const uint16_t
                                                               kslice, n_tiles, m_blocks, ks, 0, tbg, QkvRope{});
 }
 
-// Whether the wide tier takes a launch (ns == 0: no) and its configuration.  c_ok: the output's row stride
-// allows the tier's 4-element stores.
+// Whether a bf16 output takes 4-element stores: whole 8-byte rows from an 8-byte aligned base (no output: nothing to
+// store).  The wide and the many-token tier store 4 elements at a time; any other output (the head accepts every row
+// stride >= N) is the decode kernel's, which stores single elements.
+static bool c_stores4(const void* C, long ldc) { return C == nullptr || (ldc % 4 == 0 && (uintptr_t)C % 8 == 0); }
+
+// Whether the wide tier takes a launch (ns == 0: no) and its configuration.  c_ok: c_stores4 of the output.
 static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_ok) {
   const WideCfg none{0, 0, 0, 0};
   if (M <= 64 || ks <= 0) return none;
@@ -1023,8 +1027,9 @@ static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_o
 // from LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's (its cost in us: fitted to the same
 // measurements, within 25 %).  Cold weights, 8B shape at 288 / 512 rows: qkv 48 / 54 us against the wide tier's 46 / 59,
 // w13 109 / 143 against 105 / 179, w2 63 / 67 against 51 / 87.
-static DeepCfg deep_plan(int epi, int M, int N, int K, int ks) {
+static DeepCfg deep_plan(int epi, int M, int N, int K, int ks, bool c_ok) {
   const DeepCfg none{0, 0, 0, 0.0};
+  if (!c_ok) return none;
   const DeepCfg d = lsk_deep_plan(epi, M, N, K, ks);
   if (d.mg == 0 || M >= LSK_DEEP_ALWAYS_TOKENS) return d;
   double cost = 0.0;
@@ -1040,14 +1045,14 @@ static DeepCfg deep_plan(int epi, int M, int N, int K, int ks) {
   return d.us < (epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9) * us ? d : none;
 }
 
-extern "C" int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, int* cfg) {
+extern "C" int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, long ldc, int* cfg) {
   LSK_REQUIRE(cfg != nullptr, LSK_EARG, "lsk_gemm_deep_config: null pointer");
   LSK_REQUIRE(epilogue >= LSK_EPI_NONE && epilogue <= EPI_QKV, LSK_EARG, "lsk_gemm_deep_config: epilogue %d", epilogue);
   DeepCfg c{0, 0, 0, 0.0};
   if (epilogue == LSK_EPI_RESIDUAL) {
     if (lsk_gemm_residual_covers(M, N, K, ks)) c = lsk_deep_plan(epilogue, M, N, K, ks);
   } else if (epilogue != LSK_EPI_NONE) {
-    c = deep_plan(epilogue, M, N, K, ks);
+    c = deep_plan(epilogue, M, N, K, ks, epilogue == EPI_PARTIAL || epilogue == EPI_QKV || ldc % 4 == 0);
   }
   cfg[0] = c.mg;
   cfg[1] = c.m_blocks;
@@ -1070,7 +1075,7 @@ extern "C" int lsk_gemm_wide_config(int epilogue, int M, int N, int K, int ks, i
 static int launch_wide(int epi, hipStream_t s, const uint16_t* A, long lda, const uint16_t* W, uint16_t* C, long ldc,
                        const uint16_t* R, long ldr, float* P, float* av, int* ai, int M, int N, int K, int ffn, int ks,
                        bool af = false, int c_nks = 0, const QkvRope& qa = QkvRope{}) {
-  const WideCfg cfg = wide_plan(epi, M, N, K, ks, af, epi == EPI_PARTIAL || C == nullptr || ldc % 4 == 0);
+  const WideCfg cfg = wide_plan(epi, M, N, K, ks, af, c_stores4(C, ldc));
   if (cfg.ns == 0) return 0;
   const int n_tiles = N / (16 * cfg.ns);
   const dim3 grid((unsigned)(((n_tiles + 7) / 8) * 8 * cfg.m_blocks * ks));
@@ -1221,7 +1226,7 @@ extern "C" int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw
 // fragment-major too.
 static void gemm_af(int epi, hipStream_t s, const void* A, const void* W, void* C, long ldc, int c_nks, float* P,
                     float* av, int* ai, int M, int N, int K, int ffn, int ks) {
-  const DeepCfg deep = deep_plan(epi, M, N, K, ks);
+  const DeepCfg deep = deep_plan(epi, M, N, K, ks, c_stores4(C, c_nks > 0 ? 0 : ldc));
   if (deep.mg > 0) {
     lsk_gemm_deep(deep, epi, s, (const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, ldc, c_nks, nullptr, P, av, ai, M, N,
                   K, ffn, ks, QkvRope{});
@@ -1428,7 +1433,7 @@ extern "C" int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_head
   const QkvRope qa{(uint16_t*)q_out, (uint16_t*)kcache, (uint16_t*)vcache, cos_tab, sin_tab, rows, pos, n_heads,
                    n_kv_heads, head_dim, max_batch, max_seq, tab_len};
   hipStream_t s = (hipStream_t)stream;
-  const DeepCfg deep = deep_plan(EPI_QKV, M, N, K, 1);
+  const DeepCfg deep = deep_plan(EPI_QKV, M, N, K, 1, true);
   if (deep.mg > 0) {
     lsk_gemm_deep(deep, EPI_QKV, s, (const uint16_t*)A, (const uint16_t*)W, nullptr, 0, 0, nullptr, nullptr, nullptr,
                   nullptr, M, N, K, 0, 1, qa);

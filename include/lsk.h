@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define LSK_ABI_VERSION 12
+#define LSK_ABI_VERSION 13
 
 #define LSK_EPI_NONE 0     /* C = rnd(A W^T)                                   */
 #define LSK_EPI_RESIDUAL 1 /* C = rnd(R + rnd(A W^T))                          */
@@ -149,8 +149,9 @@ int lsk_gemm_plan(int N, int K, int* ns_out, int* ks_out);
 
 /* The many-token tier's configuration of a fragment-major launch (epilogue as lsk_gemm_wide_config's; LSK_EPI_RESIDUAL:
  * lsk_gemm_residual_frag where the layer runner uses it): cfg = {16-token groups per workgroup (0: another tier runs
- * the launch), token blocks, workgroups sharing a tile's K slices}.  Host only. */
-int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, int* cfg);
+ * the launch), token blocks, workgroups sharing a tile's K slices}.  ldc: row stride of the bf16 output (the head's
+ * logits; the tier stores 4 elements at a time, so a stride that is no multiple of 4 is another tier's).  Host only. */
+int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, long ldc, int* cfg);
 /* Configuration the wide-M tier (the bf16 GEMM path above 64 tokens) picks for a launch: cfg[4] = {ns (16-row
  * groups per tile; 0: the tier does not take the launch), blocks, 16-token groups per block, groups per wave}.
  * epilogue: LSK_EPI_*, or 3 = K-slice partials (lsk_gemm_partial), 4 = LM head + argmax, 5 = fused qkv + RoPE +

@@ -1077,3 +1077,16 @@ def test_deep_config_covers_every_tile_and_every_token_block():
     assert lsk.gemm_deep_config(3, 1024, 4096 + 16, 4096, 4)[0] == 0
     assert lsk.gemm_deep_config(3, 1024, 4096, 4096 + 64, 1)[0] == 0
     assert lsk.gemm_deep_config(2, 1024, 64, 4096, 1)[0] == 0
+
+
+@pytest.mark.parametrize("M", [512, 901])
+def test_deep_tier_leaves_unaligned_output_rows_to_scalar_stores(M):
+    """The head takes any logits row stride >= N; the many-token tier stores 4 logits at a time, so it takes only strides
+    that are multiples of 4 (as the wide tier).  Partials and the fused qkv have no bf16 output row to align."""
+    from thesis_amd import _lsk as lsk
+
+    N, K = 128256, 4096
+    for pad, taken in ((0, True), (1, False), (2, False), (3, False), (4, True)):
+        assert (lsk.gemm_deep_config(lsk.EPI_ARGMAX, M, N, K, 1, ldc=N + pad)[0] > 0) == taken, pad
+    assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, 901, 4096, 4096, 4, ldc=0)[0] > 0
+    assert lsk.gemm_deep_config(lsk.EPI_QKV_ROPE, 901, 6144, 4096, 1, ldc=0)[0] > 0

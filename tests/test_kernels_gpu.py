@@ -816,6 +816,27 @@ def test_many_token_gemms_are_bitwise_the_decode_kernel(cuda, M, N, K, ks):
         assert torch.equal(ids[lo:hi], i1) and torch.equal(lo_[lo:hi], l1)
 
 
+@pytest.mark.parametrize("pad,first", [(1, 0), (3, 0), (4, 0), (4, 1), (4, 2)])
+@pytest.mark.parametrize("M", [60, 100, 300, 901])
+def test_head_logits_rows_of_any_stride_and_base(cuda, M, pad, first):
+    """Logits rows of a stride or a first element that is no multiple of 4 (8 bytes): in every tier (decode, wide,
+    many-token) the ids and logits are bitwise those of contiguous rows, and nothing beside the rows is written."""
+    lsk = _lsk()
+    N, K = 12288, 256
+    g = _gen(M + pad + first)
+    h = torch.randn(M, K, generator=g).to(BF16).to(cuda)
+    w = lsk.PackedWeight((torch.randn(N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    nw = torch.ones(K, dtype=BF16, device=cuda)
+    ids, want = torch.empty(M, dtype=torch.long, device=cuda), torch.empty(M, N, dtype=BF16, device=cuda)
+    lsk.head_norm_argmax(h, nw, 1e-5, w, ids, logits=want)
+    buf = torch.full((M, N + pad), 7.0, dtype=BF16, device=cuda)
+    got, i2 = buf[:, first:first + N], torch.empty_like(ids)
+    assert got.stride(0) == N + pad and (got.data_ptr() - buf.data_ptr()) == 2 * first
+    lsk.head_norm_argmax(h, nw, 1e-5, w, i2, logits=got)
+    assert torch.equal(i2, ids) and torch.equal(got, want)
+    assert (buf[:, :first] == 7.0).all() and (buf[:, first + N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("split", [4096, 128])
 def test_shifted_segment_metadata_equals_a_plan_at_the_actual_positions(cuda, split):
     """A decode segment planned at its verifiers' upper-bound positions (all drafts accepted) and moved back on the

@@ -22,7 +22,7 @@ EPI_NONE, EPI_RESIDUAL, EPI_SILU_MUL = 0, 1, 2
 EPI_PARTIAL, EPI_ARGMAX, EPI_QKV_ROPE = 3, 4, 5   # launch kinds known to lsk_gemm_wide_config
 ATTN_SPLIT = 8192         # LSK_ATTN_SPLIT
 ATTN_ROWS = 48            # query rows per attention work item (csrc/lsk_attention.hip ATTN_ROWS)
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 # name -> (restype, argtypes)
 _P, _I, _L, _F, _Z = ctypes.c_void_p, ctypes.c_int, ctypes.c_long, ctypes.c_float, ctypes.c_size_t
@@ -50,7 +50,7 @@ _SIGS = {
     "lsk_gemm": (_I, [_I, _P, _L, _P, _L, _P, _L, _P, _L, _I, _I, _I, _I, _I, _P]),
     "lsk_gemm_plan": (_I, [_I, _I, _P, _P]),
     "lsk_gemm_wide_config": (_I, [_I, _I, _I, _I, _I, _I, _P]),
-    "lsk_gemm_deep_config": (_I, [_I, _I, _I, _I, _I, _P]),
+    "lsk_gemm_deep_config": (_I, [_I, _I, _I, _I, _I, _L, _P]),
     "lsk_gemm_partial": (_I, [_P, _L, _P, _L, _P, _I, _I, _I, _I, _P]),
     "lsk_head_workspace_bytes": (_Z, [_I, _I]),
     "lsk_head_argmax": (_I, [_I, _P, _L, _P, _L, _I, _I, _I, _P, _L, _P, _P, _P, _Z, _P]),
@@ -613,10 +613,11 @@ def gemm_wide_config(epilogue: int, M: int, N: int, K: int, ks: int = 1, af: boo
     return tuple(cfg)
 
 
-def gemm_deep_config(epilogue: int, M: int, N: int, K: int, ks: int = 1) -> tuple:
-    """(groups, token blocks, split) of a fragment-major launch in the many-token tier; groups 0: another tier."""
+def gemm_deep_config(epilogue: int, M: int, N: int, K: int, ks: int = 1, ldc: int | None = None) -> tuple:
+    """(groups, token blocks, split) of a fragment-major launch in the many-token tier; groups 0: another tier.
+    ldc: row stride of the output (None: contiguous)."""
     cfg = (ctypes.c_int * 3)()
-    _check(load().lsk_gemm_deep_config(epilogue, M, N, K, ks, cfg), "lsk_gemm_deep_config")
+    _check(load().lsk_gemm_deep_config(epilogue, M, N, K, ks, N if ldc is None else ldc, cfg), "lsk_gemm_deep_config")
     return tuple(cfg)
 
 
