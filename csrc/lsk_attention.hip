@@ -434,8 +434,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int32_t* __rest
 // wave per query row, the row's positions 0..qpos in 64-position chunks (lane = position), online softmax with
 // lsk_exp, O[d] accumulated over the chunk's positions in order.  Fixed order per query -> batch invariant.
 // Bound by the chain of a row (D dependent adds of the scores, 64 of the outputs per chunk): every row of a work item
-// has a wave of its own (blockIdx.z), and a chunk's K row and V columns are whole 16-byte loads issued before the
-// chains.  4 requests of 5 tokens, contexts to 192, 32 heads of 64 (1B shape) on MI355X: 98.8 -> 12.8 us; 121
+// has a wave of its own (blockIdx.z), and a chunk's K row and V columns are 16-byte loads (of caches at any fp32 address)
+// issued before the chains.  4 requests of 5 tokens, contexts to 192, 32 heads of 64 (1B shape) on MI355X: 98.8 -> 12.8 us; 121
 // prompt tokens: 78.2 -> 27.3 us (one wave walked up to 12 rows of an item, one dword per step).
 template <int D>
 __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ kc,
@@ -465,12 +465,13 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
       const int nvalid = min(64, qpos + 1 - base);
       // V of the chunk (first 64 d): this lane's d, 32-position blocks that hold a valid position
       const float* vb = vc + head_base + (long)base * D;
-      float4 v0[16];
+      lsk_f32x4 v0[16];
       auto load_v = [&](int d) {
 #pragma unroll
         for (int j = 0; j < 16; ++j)
-          v0[j] = d < D && 32 * (j / 8) < nvalid ? *(const float4*)(vb + (long)(j / 8) * 32 * D + d * 32 + 4 * (j % 8))
-                                                 : make_float4(0.f, 0.f, 0.f, 0.f);
+          v0[j] = d < D && 32 * (j / 8) < nvalid
+                      ? *(const lsk_f32x4_u*)(vb + (long)(j / 8) * 32 * D + d * 32 + 4 * (j % 8))
+                      : (lsk_f32x4){0.f, 0.f, 0.f, 0.f};
       };
       load_v(lane);
       float s = -INFINITY;
@@ -479,15 +480,15 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
         float acc = 0.f;
 #pragma unroll
         for (int d0 = 0; d0 < D; d0 += KB) {
-          float4 k4[KB / 4];
+          lsk_f32x4 k4[KB / 4];
 #pragma unroll
-          for (int i = 0; i < KB / 4; ++i) k4[i] = *(const float4*)(kr + d0 + 4 * i);
+          for (int i = 0; i < KB / 4; ++i) k4[i] = *(const lsk_f32x4_u*)(kr + d0 + 4 * i);
 #pragma unroll
           for (int i = 0; i < KB / 4; ++i) {
-            acc += qv[d0 + 4 * i] * k4[i].x;
-            acc += qv[d0 + 4 * i + 1] * k4[i].y;
-            acc += qv[d0 + 4 * i + 2] * k4[i].z;
-            acc += qv[d0 + 4 * i + 3] * k4[i].w;
+            acc += qv[d0 + 4 * i] * k4[i][0];
+            acc += qv[d0 + 4 * i + 1] * k4[i][1];
+            acc += qv[d0 + 4 * i + 2] * k4[i][2];
+            acc += qv[d0 + 4 * i + 3] * k4[i][3];
           }
         }
         s = acc * scale;
@@ -514,10 +515,10 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           const float4 p4 = *(const float4*)(&sp[wave][4 * j]);
-          step(4 * j, p4.x, v0[j].x);
-          step(4 * j + 1, p4.y, v0[j].y);
-          step(4 * j + 2, p4.z, v0[j].z);
-          step(4 * j + 3, p4.w, v0[j].w);
+          step(4 * j, p4.x, v0[j][0]);
+          step(4 * j + 1, p4.y, v0[j][1]);
+          step(4 * j + 2, p4.z, v0[j][2]);
+          step(4 * j + 3, p4.w, v0[j][3]);
         }
         o[i] = acc;
       }

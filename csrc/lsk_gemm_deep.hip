@@ -18,14 +18,14 @@
 
 // Rounding through bf16 by the hardware conversion: f2bf's result for every number (a NaN stays one).
 __device__ __forceinline__ float hbf(float f) { return (float)(__bf16)f; }
-__device__ __forceinline__ uint2 pack4(const float* v) {
+__device__ __forceinline__ lsk_u32x2_u pack4(const float* v) {
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   const bf16x4 b = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-  return __builtin_bit_cast(uint2, b);
+  return __builtin_bit_cast(lsk_u32x2_u, b);
 }
 
 // qkv_rope_store for rows w16 .. w16 + 3 (w16 % 4 == 0) of the pair of row groups: four consecutive dims of a head, so
-// the table rows are read and the q / K values stored 8 and 16 bytes at a time.
+// the table rows are read and the q / K values stored 16 and 8 bytes at a time (at any address their elements align).
 __device__ __forceinline__ void qkv_rope_store4(const QkvRope& qa, int m, int row, int p, int G, int w16, const float* lo,
                                                 const float* hi) {
   const int D = qa.d, GH = D >> 4, half = D >> 1;
@@ -35,10 +35,8 @@ __device__ __forceinline__ void qkv_rope_store4(const QkvRope& qa, int m, int ro
     const int h = G / GH, d1 = 16 * ((G - h * GH) >> 1) + w16;
     const float* ct = qa.cos_tab + (long)p * D + d1;
     const float* st = qa.sin_tab + (long)p * D + d1;
-    const float4 c1 = *(const float4*)ct, c2 = *(const float4*)(ct + half);
-    const float4 s1 = *(const float4*)st, s2 = *(const float4*)(st + half);
-    const float cv1[4] = {c1.x, c1.y, c1.z, c1.w}, cv2[4] = {c2.x, c2.y, c2.z, c2.w};
-    const float sv1[4] = {s1.x, s1.y, s1.z, s1.w}, sv2[4] = {s2.x, s2.y, s2.z, s2.w};
+    const lsk_f32x4 cv1 = *(const lsk_f32x4_u*)ct, cv2 = *(const lsk_f32x4_u*)(ct + half);
+    const lsk_f32x4 sv1 = *(const lsk_f32x4_u*)st, sv2 = *(const lsk_f32x4_u*)(st + half);
     float o1[4], o2[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // rope_pair's roundings
@@ -54,8 +52,8 @@ __device__ __forceinline__ void qkv_rope_store4(const QkvRope& qa, int m, int ro
       dst1 = base + k_cache_offset<uint16_t>(p, d1, D);
       dst2 = base + k_cache_offset<uint16_t>(p, d1 + half, D);
     }
-    *(uint2*)dst1 = pack4(o1);
-    *(uint2*)dst2 = pack4(o2);
+    *(lsk_u32x2_u*)dst1 = pack4(o1);
+    *(lsk_u32x2_u*)dst2 = pack4(o2);
   } else {
     const int gv = G - kg, h = gv / GH, d1 = 16 * (gv - h * GH) + w16;
     uint16_t* dst = qa.vc + ((long)row * qa.hkv + h) * (long)D * qa.max_seq + (long)(p >> 5) * 32 * D + (p & 31);
@@ -308,8 +306,7 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           o[i] = hbf(silu_f(hbf(tot[g][t][i] + empty))) * hbf(tot[g + WN][t][i] + empty);
-        const uint2 pk = pack4(o);
-        *(uint2*)(C + (c_nks > 0 ? lsk_frag_off(m, n, c_nks) : (long)m * ldc + n)) = pk;
+        *(lsk_u32x2_u*)(C + (c_nks > 0 ? lsk_frag_off(m, n, c_nks) : (long)m * ldc + n)) = pack4(o);
       }
     }
   } else if constexpr (EPI == EPI_QKV) {
@@ -337,13 +334,13 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
         const long off = (long)m * ldc + (r0 + g) * 16 + 4 * lg;
-        const uint2 x = *(const uint2*)(R + off);
+        const lsk_u32x2_u x = *(const lsk_u32x2_u*)(R + off);
         float o[4] = {__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16),
                       __uint_as_float(x.y & 0xffff0000u)};
         const lsk_f32x4 v = sums[(g * MG + t) * 256];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = o[i] + hbf(v[i]);
-        *(uint2*)(C + off) = pack4(o);
+        *(lsk_u32x2_u*)(C + off) = pack4(o);
       }
     }
   } else if constexpr (EPI == EPI_ARGMAX) {

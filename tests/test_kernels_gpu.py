@@ -381,6 +381,30 @@ def test_ragged_attention_f32_is_bitwise_the_ordered_one(cuda, D, Hq, Hkv):
         assert np.array_equal(got.numpy(), want), cap
 
 
+def _shifted(t, by):
+    """A contiguous copy of t that starts `by` elements into its (16-byte aligned) allocation."""
+    out = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)[by:].view(t.shape)
+    assert out.is_contiguous() and out.data_ptr() % 16 == by * t.element_size() % 16
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("D", [16, 64, 128])
+def test_ragged_attention_f32_reads_caches_at_any_fp32_address(cuda, D):
+    """q, K and V one, two or three floats past a 16-byte boundary: the same bits as aligned ones."""
+    lsk = _lsk()
+    q, kc, vc, tab, _ = _attn_case(D + 1, F32, 2, 4, 2, D, 128, [(0, 0, 3), (1, 90, 5)])
+    works, _, _ = lsk.attn_plan(tab, 2, 1 << 30, 16)
+    qd, kd, vd = q.to(cuda), kc.to(cuda), lsk.v_to_blocked(vc).to(cuda)
+    td, wd = torch.from_numpy(tab).to(cuda), torch.from_numpy(works).to(cuda)
+    outs = []
+    for by in range(4):
+        out = torch.empty(q.shape[0], 4 * D, device=cuda)
+        lsk.ragged_attn(_shifted(qd, by), _shifted(kd, by), _shifted(vd, by), td, wd, len(works), None, 0, 0, out, 4,
+                        1.0 / math.sqrt(D), rows_cap=16)
+        outs.append(out)
+    assert all(torch.equal(o, outs[0]) for o in outs)
+
+
 def test_ragged_attention_bf16_is_batch_invariant(cuda):
     """A query's output is bitwise the same alone (T = 1) and inside a verify block that crosses a
     split boundary."""
@@ -929,6 +953,31 @@ def test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, heads):
     assert torch.equal(k2.view(torch.int16), k1.view(torch.int16))
     assert torch.equal(v2.view(torch.int16), v1.view(torch.int16))
     assert not torch.equal(k2, k0) and not torch.equal(v2, v0)
+
+
+@pytest.mark.parametrize("M", [8, 100, 1200])
+def test_fused_qkv_at_addresses_only_their_elements_align(cuda, M):
+    """RoPE tables, q and caches one to three elements past a 16-byte boundary, in the decode, wide and many-token
+    tiers: the same bits as aligned ones."""
+    lsk = _lsk()
+    heads, K, B, S = (8, 8, 64), 512, 2, 1024
+    Hq, Hkv, D = heads
+    assert (lsk.gemm_deep_config(lsk.EPI_QKV_ROPE, M, (Hq + 2 * Hkv) * D, K)[0] > 0) == (M == 1200)
+    g = _gen(M)
+    af = lsk.PackedWeight(torch.randn(lsk.frag_rows(M), K, generator=g).to(BF16).to(cuda)).data
+    w = lsk.PackedWeight((torch.randn((Hq + 2 * Hkv) * D, K, generator=g) * 0.05).to(BF16).to(cuda), qkv_heads=heads)
+    cos, sin = torch.randn(S, D, generator=g).to(cuda), torch.randn(S, D, generator=g).to(cuda)
+    perm = torch.randperm(B * S, generator=g)[:M]
+    rows, pos = (perm // S).to(torch.int32).to(cuda), (perm % S).to(torch.int32).to(cuda)
+    res = []
+    for by in range(4):
+        q = _shifted(torch.zeros(M, Hq, D, dtype=BF16, device=cuda), by)
+        k = _shifted(torch.zeros(B, Hkv, S // 32, D // 16, 64, 8, dtype=BF16, device=cuda), by)
+        v = _shifted(torch.zeros(B, Hkv, S // 32, D, 32, dtype=BF16, device=cuda), by)
+        lsk.gemm_qkv_rope(af, w, M, q, k, v, _shifted(cos, by), _shifted(sin, by), rows, pos)
+        res.append((q, k, v))
+    assert all(torch.equal(a, b) for r in res for a, b in zip(r, res[0]))
+    assert all((t != 0).any() for t in res[0])
 
 
 @pytest.mark.parametrize("M", [1, 15, 16, 17])
