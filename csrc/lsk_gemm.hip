@@ -1447,9 +1447,12 @@ extern "C" int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_head
     // tokens 11.9 -> 10.0 us on MI355X
     const int mr = M - mw;
     int ms = ms_for(mr);
-    // up to 16 tokens such a weight runs half-width tiles (8 rotation pairs, twice the workgroups): a 1B decode step of one
-    // token 270.5 -> 265.3 us over 6 layers; with 192 tiles or more they are slower (8B shape 11.8 -> 13.7 us a launch)
-    const int ns = N / 32 < 192 && mr <= 16 ? 1 : 2;
+    // up to 16 tokens half-width tiles (8 rotation pairs, twice the workgroups) where they still start in one round, at
+    // most one per CU: 16 / 48 / 96 / 128 tiles of 32 rows 6.3 / 6.6 / 7.0 / 7.4 -> 5.4 / 5.7 / 6.1 / 6.4 us (K = 2048, one
+    // to 16 tokens alike; K = 4096 with 96 / 128 tiles 10.9 / 11.5 -> 9.1 / 9.9); from 160 tiles on the second round costs
+    // more than it gives (160 / 192 / 256: 7.7 / 8.1 / 9.0 -> 8.4 / 8.7 / 9.4, K = 4096 12.0 / 12.6 / 14.5 -> 13.9 / 14.8 /
+    // 16.1; 384: within 3 %).  Cold weights, graph-timed.
+    const int ns = N / 16 <= 256 && mr <= 16 ? 1 : 2;
     while (ms > 1 && (long)(N / 32) * ((mr + 16 * ms - 1) / (16 * ms)) < 192) --ms;
     dispatch_bf16(ns, ms, EPI_QKV, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, 0, W, K, nullptr, 0, nullptr, 0,
                   nullptr, nullptr, nullptr, M, N, K, 0, K, true, mw, 0, qa);

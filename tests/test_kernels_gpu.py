@@ -980,8 +980,9 @@ def test_fused_qkv_at_addresses_only_their_elements_align(cuda, M):
     assert all((t != 0).any() for t in res[0])
 
 
-@pytest.mark.parametrize("M", [1, 15, 16, 17])
-def test_fused_qkv_half_width_tiles(cuda, M):
-    """Weights of fewer than 192 32-row tiles run half-width tiles (8 rotation pairs each) up to 16 tokens: the same
-    writes as the unfused path on both sides of that line, q, k and v rows alike."""
-    test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, (8, 2, 64))
+@pytest.mark.parametrize("M,heads", [(1, (8, 2, 64)), (15, (8, 2, 64)), (16, (8, 2, 64)), (17, (8, 2, 64)),
+                                     (16, (32, 16, 64)), (16, (34, 17, 64))])
+def test_fused_qkv_half_width_tiles(cuda, M, heads):
+    """Weights of up to 128 32-row tiles run half-width tiles (8 rotation pairs each) up to 16 tokens: the same
+    writes as the unfused path on both sides of both lines, q, k and v rows alike."""
+    test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, heads)
