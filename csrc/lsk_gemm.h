@@ -55,7 +55,7 @@ __device__ __forceinline__ void qkv_rope_store(const QkvRope& qa, int m, int G, 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + lsk_exp(-x)); }
 
 #define LSK_DEEP_MIN_TOKENS 256     // below: the wide tier
-#define LSK_DEEP_ALWAYS_TOKENS 900  // from here on: the many-token tier whatever the estimates
+#define LSK_DEEP_ALWAYS_TOKENS 900  // from here on the many-token tier unless its estimate is the higher one
 // Many-token tier (lsk_gemm_deep.hip) over a fragment-major A: whether it takes a launch, and the launch.  Same sums as
 // the other tiers.
 struct DeepCfg {
@@ -63,7 +63,6 @@ struct DeepCfg {
   double us;                // estimated time
 };
 DeepCfg lsk_deep_plan(int epi, int M, int N, int K, int ks);
-bool lsk_deep_sums(int M, int N, int K, int ks);
 void lsk_gemm_deep(const DeepCfg& cfg, int epi, hipStream_t s, const uint16_t* A, const uint16_t* W, uint16_t* C, long ldc,
                    int c_nks, const uint16_t* R, float* P, float* av, int* ai, int M, int N, int K, int ffn, int ks,
                    const QkvRope& qa);

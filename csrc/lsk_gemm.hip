@@ -1022,27 +1022,50 @@ static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_o
   return wide_config(epi, M, N, ks);
 }
 
-// The many-token tier's configuration where it takes a fragment-major launch (mg == 0: it does not).  From
-// LSK_DEEP_ALWAYS_TOKENS rows on it always does (faster or within 5 % at every projection of the 1B, 7B and 8B shapes);
-// from LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's (its cost in us: fitted to the same
-// measurements, within 25 %).  Cold weights, 8B shape at 288 / 512 rows: qkv 48 / 54 us against the wide tier's 46 / 59,
-// w13 109 / 143 against 105 / 179, w2 63 / 67 against 51 / 87.
+// The wide tier's estimated time (us) of a launch it takes: its cost fitted to measurements over the presets' projections
+// (within 25 %; the presets' heads and launches of two or more rounds scatter most).
+static double wide_us(int epi, int M, int N, int K, int ks) {
+  double cost = 0.0;
+  wide_config(epi, M, N, ks, &cost);
+  cost *= (double)(K / ks) / 4096.0;
+  if (epi == LSK_EPI_SILU_MUL) return 15.8 * cost + 9.0;
+  if (epi == EPI_PARTIAL) return 7.4 * cost + 4.5 + 2.0 * ks * (double)M * N * 4.0 / 4.5e6;
+  return 11.1 * cost + 4.5;
+}
+
+// The many-token tier's configuration where it takes a fragment-major launch (mg == 0: it does not; c_ok: c_stores4 of
+// the output).  Times: MI355X, cold weights, graph-timed; partials with the norm that adds them.
+// * Few weight tiles (wide_plan takes nothing): the decode tier's small workgroups fill the chip where 15-60 workgroups of
+//   256 rows leave it idle: qkv 512 x 512 at 900 / 1517 tokens 6.5 / 8.5 us against 13.1 / 13.3, silu-mul 256 x 1024 8.0 / 8.6
+//   against 14.9 / 15.1, partials 768 x 768 14.6 / 19.3 against 20.5 / 23.7.  From three rounds of its 32 x 64-token tiles
+//   and K > 1024 on it is the slower one (qkv 512 x 2048 at 2100 tokens 32.1 against 23.9, silu-mul 30.0 against 22.5), and
+//   for the head (2048 x 1024 with logits at 900 / 1517 tokens 28.9 / 28.1 against 22.8 / 25.4).
+// * From LSK_DEEP_ALWAYS_TOKENS rows on always for qkv and the head (3-50 % faster over 69 and 14 launches of small and
+//   preset shapes, two within 4 %); partials where its estimate is the lower one (512 x 512 at 1517: 17.2 against 19.8,
+//   the presets' 11 % slower to 61 % faster); silu-mul up to 1.15 times the wide tier's estimate, which is the low one
+//   where it plans two rounds (1408 x 2048 at 900: 22.8 against 28.4 us, left to the wide tier; at 2100: 83.6 against 35.4).
+// * From LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's.  8B shape at 304 / 512 rows: qkv
+//   54.6 / 55.5 us against the wide tier's 46.7 / 58.2, w13 116 / 144 against 108 / 174, w2 74 / 82 against 62 / 97.
 static DeepCfg deep_plan(int epi, int M, int N, int K, int ks, bool c_ok) {
   const DeepCfg none{0, 0, 0, 0.0};
   if (!c_ok) return none;
   const DeepCfg d = lsk_deep_plan(epi, M, N, K, ks);
-  if (d.mg == 0 || M >= LSK_DEEP_ALWAYS_TOKENS) return d;
-  double cost = 0.0;
-  if (wide_plan(epi, M, N, K, ks, true, true).ns == 0) return none;  // (few weight tiles: the decode tier)
-  if (epi == EPI_PARTIAL && K / ks < 512) return none;               // a class per chunk: folds and stores dominate
-  wide_config(epi, M, N, ks, &cost);
-  cost *= (double)(K / ks) / 4096.0;
-  double us;
-  if (epi == LSK_EPI_SILU_MUL) us = 15.8 * cost + 9.0;
-  else if (epi == EPI_PARTIAL) us = 7.4 * cost + 4.5 + 2.0 * ks * (double)M * N * 4.0 / 4.5e6;
-  else us = 11.1 * cost + 4.5;
-  // the partials' and the head's estimates scatter more
-  return d.us < (epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9) * us ? d : none;
+  if (d.mg == 0) return none;
+  const bool many = M >= LSK_DEEP_ALWAYS_TOKENS;
+  if (wide_plan(epi, M, N, K, ks, true, true).ns == 0) {
+    const long rounds = ((long)(N / 32) * ((M + 63) / 64) + 255) / 256;
+    const bool faster = epi == EPI_ARGMAX || (epi != EPI_PARTIAL && rounds >= 3 && K > 1024);
+    return many && faster ? d : none;
+  }
+  if (!many && epi == EPI_PARTIAL && K / ks < 512) return none;  // a class per chunk: folds and stores dominate
+  double f;
+  if (many) {
+    if (epi == EPI_QKV || epi == EPI_ARGMAX) return d;
+    f = epi == EPI_PARTIAL ? 1.0 : 1.15;
+  } else {
+    f = epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9;  // the partials' and the head's estimates scatter more
+  }
+  return d.us < f * wide_us(epi, M, N, K, ks) ? d : none;
 }
 
 extern "C" int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, long ldc, int* cfg) {
@@ -1262,9 +1285,15 @@ int lsk_gemm_silu_af(const void* A, const void* W, void* H, int h_frag, int M, i
 }
 
 // Whether the o / w2 projection of M rows sums its K slices in the GEMM (lsk_gemm_residual_frag) instead of leaving
-// partials for the next add + RMSNorm.
+// partials for the next add + RMSNorm to read: where that saves more than walking all slices in one workgroup costs (its
+// estimate is about a tenth low).  With the norm, o of the 8B shape at 1000 / 1517 / 4001 tokens 67 / 78 / 188 us against
+// 67 / 101 / 277 as partials, w2 186 / 198 / 450 against 139 / 226 / 551; 512 x 2048 in 16 slices at 1517 tokens 47.8
+// against 34.1.  A weight of few tiles stays the decode tier's.
 bool lsk_gemm_residual_covers(int M, int N, int K, int ks) {
-  return M >= LSK_DEEP_ALWAYS_TOKENS && lsk_deep_sums(M, N, K, ks);
+  if (M < LSK_DEEP_ALWAYS_TOKENS || wide_plan(EPI_PARTIAL, M, N, K, ks, true, true).ns == 0) return false;
+  const DeepCfg r = lsk_deep_plan(LSK_EPI_RESIDUAL, M, N, K, ks), p = deep_plan(EPI_PARTIAL, M, N, K, ks, true);
+  const double p_us = p.mg > 0 ? p.us : wide_us(EPI_PARTIAL, M, N, K, ks);
+  return r.mg > 0 && 1.1 * r.us <= p_us + ks * (double)M * N * 4.0 / 4.5e6;
 }
 
 extern "C" int lsk_gemm_residual_frag(const void* A, const void* W, const void* R, void* C, int M, int N, int K, int ks,

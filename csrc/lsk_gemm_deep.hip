@@ -392,8 +392,8 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
 // projections at 256-4001 tokens:
 //   mg = 8 / 6 (one workgroup per CU): 1.7 c + 12 (a single round: 6 with partials, else 14) / 1.25 c + 13 us each (mg = 6: 1.4 c up to
 //     1024 tokens)
-//   mg = 4 (two per CU): 2.1 c + 3 us per pair (2.5 c up to 1024 tokens and with partials), a lone one 1.3 c + 10 us
-//     (1.5 c + 9 summing its slices)
+//   mg = 4 (two per CU): 2.1 c + 3 us per pair (2.5 c up to 1024 tokens and with partials, 2.5 c + 8 for the LM head), a
+//     lone one 1.3 c + 10 us (1.5 c + 9 summing its slices)
 // plus 3 us per slice summed, plus the stores of the partials.  Larger mg moves fewer bytes per product (24, 22 and 20 KiB
 // per k-step for 8, 6 and 4 x 16 tokens of 256 rows), smaller mg splits a segment into more workgroups and overlaps one
 // workgroup's epilogue with the other's products: w13 of the 8B shape at 4001 tokens 920 / 992 / 943 us, at 512 tokens
@@ -401,6 +401,7 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
 DeepCfg lsk_deep_plan(int epi, int M, int N, int K, int ks) {
   const DeepCfg none{0, 0, 0, 0.0};
   const bool silu = epi == LSK_EPI_SILU_MUL, partial = epi == EPI_PARTIAL, sum = epi == LSK_EPI_RESIDUAL;
+  const bool head = epi == EPI_ARGMAX;
   const int cols = silu ? 128 : 256;
   if (M < LSK_DEEP_MIN_TOKENS || ks < 1 || N % cols != 0 || K % ks != 0 || (K / ks) % 128 != 0) return none;
   // 32-bit byte offsets into both operands
@@ -417,7 +418,8 @@ DeepCfg lsk_deep_plan(int epi, int M, int N, int K, int ks) {
       double us;
       if (mg == 4) {
         const double lone = sum ? 1.5 * c + 9.0 : 1.3 * c + 10.0;
-        us = (n / 2) * ((partial || M <= 1024 ? 2.5 : 2.1) * c + 3.0 + (sum ? 2.5 * ks : 0.0)) + (n & 1 ? lone : 0.0);
+        const double pair = (partial || head || M <= 1024 ? 2.5 : 2.1) * c + (head ? 8.0 : 3.0) + (sum ? 2.5 * ks : 0.0);
+        us = (n / 2) * pair + (n & 1 ? lone : 0.0);
       } else {
         us = n * (mg == 8 ? 1.7 * c + (n > 1 ? 12.0 : (partial ? 6.0 : 14.0)) : (M <= 1024 ? 1.4 : 1.25) * c + 13.0) +
              (sum ? 3.0 * ks * n : 0.0);
@@ -427,14 +429,6 @@ DeepCfg lsk_deep_plan(int epi, int M, int N, int K, int ks) {
     }
   }
   return best;
-}
-
-// Whether summing the K slices in the launch beats leaving partials for the next add + RMSNorm to read (o of the 8B shape
-// with its norm at 768 / 1517 / 4001 tokens: 54 / 72 / 180 us against 51 / 99 / 271; w2 189 / 196 / 446 at 1024 / 1517 /
-// 4001 against 136 / 223 / 542).
-bool lsk_deep_sums(int M, int N, int K, int ks) {
-  const DeepCfg r = lsk_deep_plan(LSK_EPI_RESIDUAL, M, N, K, ks), p = lsk_deep_plan(EPI_PARTIAL, M, N, K, ks);
-  return r.mg > 0 && r.us <= p.us + ks * (double)M * N * 4.0 / 4.5e6;
 }
 
 void lsk_gemm_deep(const DeepCfg& cfg, int epi, hipStream_t s, const uint16_t* A, const uint16_t* W, uint16_t* C, long ldc,

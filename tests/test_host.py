@@ -1079,6 +1079,29 @@ def test_deep_config_covers_every_tile_and_every_token_block():
     assert lsk.gemm_deep_config(2, 1024, 64, 4096, 1)[0] == 0
 
 
+def test_deep_tier_leaves_weights_of_few_tiles_to_the_decode_tier():
+    """A small weight gives the many-token tier too few workgroups of 256 rows: at any token count its launches stay where
+    they are faster, and its o / w2 keep their partials; the presets' projections take the tier as before."""
+    from thesis_amd import _lsk as lsk
+
+    for M in (900, 1517):
+        for epi, N, K in ((lsk.EPI_QKV_ROPE, 512, 512), (lsk.EPI_QKV_ROPE, 512, 1024), (lsk.EPI_SILU_MUL, 256, 1024),
+                          (lsk.EPI_SILU_MUL, 512, 2048), (lsk.EPI_PARTIAL, 768, 768), (lsk.EPI_RESIDUAL, 768, 768),
+                          (lsk.EPI_PARTIAL, 256, 256), (lsk.EPI_RESIDUAL, 256, 256)):
+            ks = lsk.gemm_plan(N, K)[1] if epi in (lsk.EPI_PARTIAL, lsk.EPI_RESIDUAL) else 1
+            assert lsk.gemm_deep_config(epi, M, N, K, ks)[0] == 0, (M, epi, N, K)
+    assert lsk.gemm_deep_config(lsk.EPI_RESIDUAL, 1517, 512, 2048, 16)[0] == 0       # summing 16 slices costs more
+    for dim, qkv, ffn, ks in ((2048, 3072, 8192, 8), (4096, 6144, 14336, 4), (4096, 12288, 11008, 2)):
+        for M in (900, 1517, 4001):
+            assert lsk.gemm_deep_config(lsk.EPI_QKV_ROPE, M, qkv, dim)[0] > 0
+            assert lsk.gemm_deep_config(lsk.EPI_SILU_MUL, M, ffn, dim)[0] > 0
+            assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, M, dim, ffn, ks)[0] > 0
+        assert lsk.gemm_deep_config(lsk.EPI_RESIDUAL, 1517, dim, dim, 8 if dim == 2048 else 4)[0] > 0
+        assert lsk.gemm_deep_config(lsk.EPI_RESIDUAL, 4001, dim, ffn, ks)[0] > 0
+    # the 1B head at 1152 rows: 8 token groups a workgroup (746 us; 4 groups 887, the wide tier 824)
+    assert lsk.gemm_deep_config(lsk.EPI_ARGMAX, 1152, 128256, 2048)[0] == 8
+
+
 @pytest.mark.parametrize("M", [512, 901])
 def test_deep_tier_leaves_unaligned_output_rows_to_scalar_stores(M):
     """The head takes any logits row stride >= N; the many-token tier stores 4 logits at a time, so it takes only strides

@@ -799,45 +799,97 @@ def test_small_token_tiles_are_bitwise_the_wider_ones(cuda, ffn, K):
         assert torch.equal(lsk.gemm_partial(x, w, ks), part[:, :m]), m
 
 
-@pytest.mark.parametrize("M,N,K,ks", [(256, 8192, 1024, 1), (900, 256, 128, 1), (901, 512, 512, 4), (911, 2048, 2048, 8),
-                                      (930, 4096, 1024, 4), (1025, 1024, 1536, 2), (1100, 8192, 512, 1),
-                                      (2000, 4096, 768, 1), (2049, 2048, 1280, 2)])
-def test_many_token_gemms_are_bitwise_the_decode_kernel(cuda, M, N, K, ks):
-    """The many-token tier (4, 6 and 8 token groups per workgroup, slices split over workgroups or summed in one, chunk
-    classes with and without chunks, ragged last groups): partials, silu-mul (row- and fragment-major), residual and
-    the head's logits and ids are bitwise those of 64-row (decode tier) launches over the same rows."""
+# (launch kind, M, N, K, K slices, 16-token groups per workgroup).  Every kind at 4, 6 and 8 groups, either side of 900
+# tokens, mostly with a ragged last group and blocks of unequal group counts; slices of one to four and more chunks.
+MANY_TOKEN_CASES = [
+    ("partial", 257, 3072, 4096, 8, 4), ("partial", 257, 2560, 4096, 8, 8), ("partial", 850, 6144, 4096, 8, 6),
+    ("partial", 901, 512, 1024, 8, 8), ("partial", 911, 2048, 2048, 8, 8), ("partial", 1025, 2048, 768, 2, 4),
+    ("partial", 1050, 4096, 128, 1, 4), ("partial", 1400, 1536, 4096, 8, 6), ("partial", 2100, 1024, 384, 3, 8),
+    ("partial", 2700, 1536, 2048, 4, 6), ("partial", 2049, 2048, 1280, 2, 8),
+    ("silu", 333, 6144, 128, 1, 4), ("silu", 400, 8192, 2048, 1, 8), ("silu", 450, 6144, 1536, 1, 6),
+    ("silu", 901, 2560, 1280, 1, 6), ("silu", 1001, 3072, 2048, 1, 8), ("silu", 1250, 1024, 384, 1, 4),
+    ("head", 257, 12288, 2048, 1, 4), ("head", 600, 12288, 1024, 1, 8), ("head", 650, 6144, 2048, 1, 6),
+    ("head", 901, 256, 128, 1, 4), ("head", 1001, 6144, 1024, 1, 8), ("head", 2700, 1536, 512, 1, 6),
+    ("residual", 901, 6144, 1280, 2, 6), ("residual", 1001, 6144, 2048, 2, 8), ("residual", 1517, 768, 384, 3, 4),
+    ("residual", 1517, 2048, 2048, 8, 4),
+]
+
+
+@pytest.mark.parametrize("kind,M,N,K,ks,groups", MANY_TOKEN_CASES)
+def test_many_token_gemms_are_bitwise_the_decode_kernel(cuda, kind, M, N, K, ks, groups):
+    """The many-token tier at every group count of every launch kind (asserted against its own plan): partials, silu-mul
+    (row- and fragment-major), residual (in place too) and the head's logits and ids are bitwise those of 64-row (decode
+    tier) launches over the same rows.  The fused qkv has test_fused_qkv_many_token_tiles."""
     lsk = _lsk()
-    g = _gen(M + N + K)
-    m16 = lsk.frag_rows(M)
-    a = torch.randn(m16, K, generator=g).to(BF16).to(cuda)
+    code = {"partial": lsk.EPI_PARTIAL, "silu": lsk.EPI_SILU_MUL, "head": lsk.EPI_ARGMAX, "residual": lsk.EPI_RESIDUAL}
+    assert lsk.gemm_deep_config(code[kind], M, N, K, ks)[0] == groups
+    g = torch.Generator(device=cuda).manual_seed(M + N + K)
+    a = torch.randn(lsk.frag_rows(M), K, generator=g, device=cuda).to(BF16)
     af = lsk.PackedWeight(a).data
-    w = lsk.PackedWeight((torch.randn(N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    w = lsk.PackedWeight((torch.randn((2 if kind == "silu" else 1) * N, K, generator=g, device=cuda) * 0.05).to(BF16))
     parts = [(lo, min(lo + 64, M)) for lo in range(0, M, 64)]
-    want = torch.cat([lsk.gemm_partial(a[lo:hi].contiguous(), w, ks) for lo, hi in parts], dim=1)
-    assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, M, N, K, ks)[0] > 0 or M < 900
-    assert torch.equal(lsk.gemm_partial_frag(af, M, w, ks), want)
-    if lsk.gemm_deep_config(lsk.EPI_RESIDUAL, M, N, K, ks)[0]:
-        r = torch.randn(M, N, generator=g).to(BF16).to(cuda)
+    if kind in ("partial", "residual"):
+        want = torch.cat([lsk.gemm_partial(a[lo:hi].contiguous(), w, ks) for lo, hi in parts], dim=1)
+        if kind == "partial":
+            assert torch.equal(lsk.gemm_partial_frag(af, M, w, ks), want)
+            return
+        r = torch.randn(M, N, generator=g, device=cuda).to(BF16)
         x = torch.empty_like(r)
         lsk.add_rmsnorm(r, want, None, 1e-5, x_out=x)
         assert torch.equal(lsk.gemm_residual_frag(af, M, w, ks, r), x)
         assert torch.equal(lsk.gemm_residual_frag(af, M, w, ks, r, out=r), x)      # in place
-    w13 = lsk.PackedWeight((torch.randn(2 * N, K, generator=g) * 0.05).to(BF16).to(cuda))
-    want = torch.cat([lsk.gemm(a[lo:hi].contiguous(), w13, epilogue=lsk.EPI_SILU_MUL) for lo, hi in parts])
-    h = torch.empty(M, N, dtype=BF16, device=cuda)
-    assert torch.equal(lsk.gemm_silu_frag(af, M, w13, h, False), want)
-    h = torch.empty(m16 * N, dtype=BF16, device=cuda)
-    lsk.gemm_silu_frag(af, M, w13, h, True)
-    back = lsk.PackedWeight.__new__(lsk.PackedWeight)
-    back.shape, back.dtype, back.device, back.data = (m16, N), BF16, h.device, h
-    assert torch.equal(back.unpack()[:M], want)
-    nw = torch.ones(K, dtype=BF16, device=cuda)
-    ids, lo_ = torch.empty(M, dtype=torch.long, device=cuda), torch.empty(M, N, dtype=BF16, device=cuda)
-    lsk.head_norm_argmax(a[:M].contiguous(), nw, 1e-5, w, ids, logits=lo_)
-    for lo, hi in parts:
-        i1, l1 = torch.empty(hi - lo, dtype=torch.long, device=cuda), torch.empty(hi - lo, N, dtype=BF16, device=cuda)
-        lsk.head_norm_argmax(a[lo:hi].contiguous(), nw, 1e-5, w, i1, logits=l1)
-        assert torch.equal(ids[lo:hi], i1) and torch.equal(lo_[lo:hi], l1)
+    elif kind == "silu":
+        want = torch.cat([lsk.gemm(a[lo:hi].contiguous(), w, epilogue=lsk.EPI_SILU_MUL) for lo, hi in parts])
+        h = torch.empty(M, N, dtype=BF16, device=cuda)
+        assert torch.equal(lsk.gemm_silu_frag(af, M, w, h, False), want)
+        h = torch.empty(lsk.frag_rows(M) * N, dtype=BF16, device=cuda)
+        lsk.gemm_silu_frag(af, M, w, h, True)
+        back = lsk.PackedWeight.__new__(lsk.PackedWeight)
+        back.shape, back.dtype, back.device, back.data = (lsk.frag_rows(M), N), BF16, h.device, h
+        assert torch.equal(back.unpack()[:M], want)
+    else:
+        nw = torch.ones(K, dtype=BF16, device=cuda)
+        ids, got = torch.empty(M, dtype=torch.long, device=cuda), torch.empty(M, N, dtype=BF16, device=cuda)
+        lsk.head_norm_argmax(a[:M].contiguous(), nw, 1e-5, w, ids, logits=got)
+        for lo, hi in parts:
+            i1, l1 = torch.empty(hi - lo, dtype=torch.long, device=cuda), torch.empty(hi - lo, N, dtype=BF16, device=cuda)
+            lsk.head_norm_argmax(a[lo:hi].contiguous(), nw, 1e-5, w, i1, logits=l1)
+            assert torch.equal(ids[lo:hi], i1) and torch.equal(got[lo:hi], l1)
+
+
+@pytest.mark.parametrize("kind", ["partial", "silu", "residual"])
+def test_many_token_gemms_on_special_values(cuda, kind):
+    """Rows of infinities, NaN, products that overflow and that leave the normal range: the many-token tier rounds by the
+    hardware conversion where the decode kernel rounds in integers -- NaN in the same places, all else bitwise."""
+    lsk = _lsk()
+    M, N, K, ks = 1001, 4096, 512, 2
+    g = torch.Generator(device=cuda).manual_seed(5)
+    a = torch.randn(lsk.frag_rows(M), K, generator=g, device=cuda)
+    scale = torch.ones(a.shape[0], 1, device=cuda)
+    scale[0::7], scale[1::7], scale[2::7] = 2.0 ** 126, 2.0 ** -122, 2.0 ** -130
+    a = (a * scale).to(BF16)
+    a[3::7, 5], a[4::7, 9], a[5::7, 11] = float("inf"), -float("inf"), float("nan")
+    af = lsk.PackedWeight(a).data
+    w = lsk.PackedWeight((torch.randn((2 if kind == "silu" else 1) * N, K, generator=g, device=cuda) * 0.05).to(BF16))
+    parts = [(lo, min(lo + 64, M)) for lo in range(0, M, 64)]
+    if kind == "silu":
+        assert lsk.gemm_deep_config(lsk.EPI_SILU_MUL, M, N, K)[0] > 0
+        want = torch.cat([lsk.gemm(a[lo:hi].contiguous(), w, epilogue=lsk.EPI_SILU_MUL) for lo, hi in parts])
+        got = lsk.gemm_silu_frag(af, M, w, torch.empty(M, N, dtype=BF16, device=cuda), False)
+    else:
+        assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, M, N, K, ks)[0] > 0
+        want = torch.cat([lsk.gemm_partial(a[lo:hi].contiguous(), w, ks) for lo, hi in parts], dim=1)
+        if kind == "partial":
+            got = lsk.gemm_partial_frag(af, M, w, ks)
+        else:
+            r = torch.zeros(M, N, dtype=BF16, device=cuda)
+            p, want = want, torch.empty_like(r)
+            lsk.add_rmsnorm(r, p, None, 1e-5, x_out=want)
+            got = lsk.gemm_residual_frag(af, M, w, ks, r)
+    bits = torch.int32 if kind == "partial" else torch.int16
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan) and nan.any() and want.isinf().any() and not nan.all()
+    assert torch.equal(got.view(bits)[~nan], want.view(bits)[~nan])
 
 
 @pytest.mark.parametrize("pad,first", [(1, 0), (3, 0), (4, 0), (4, 1), (4, 2)])
