@@ -1087,7 +1087,11 @@ extern "C" int lsk_gemm_wide_config(int epilogue, int M, int N, int K, int ks, i
   LSK_REQUIRE(cfg != nullptr, LSK_EARG, "lsk_gemm_wide_config: null pointer");
   LSK_REQUIRE(epilogue >= LSK_EPI_NONE && epilogue <= EPI_QKV, LSK_EARG, "lsk_gemm_wide_config: epilogue %d",
               epilogue);
-  const WideCfg c = wide_plan(epilogue, M, N, K, ks, af != 0, true);
+  WideCfg c{0, 0, 0, 0};
+  // (the launch asks the many-token tier first)
+  const bool deep = af && epilogue != LSK_EPI_NONE && epilogue != LSK_EPI_RESIDUAL &&
+                    deep_plan(epilogue, M, N, K, ks, true).mg > 0;
+  if (!deep) c = wide_plan(epilogue, M, N, K, ks, af != 0, true);
   cfg[0] = c.ns;
   cfg[1] = c.m_blocks;
   cfg[2] = c.tbg;

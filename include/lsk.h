@@ -153,7 +153,7 @@ int lsk_gemm_plan(int N, int K, int* ns_out, int* ks_out);
  * logits; the tier stores 4 elements at a time, so a stride that is no multiple of 4 is another tier's).  Host only. */
 int lsk_gemm_deep_config(int epilogue, int M, int N, int K, int ks, long ldc, int* cfg);
 /* Configuration the wide-M tier (the bf16 GEMM path above 64 tokens) picks for a launch: cfg[4] = {ns (16-row
- * groups per tile; 0: the tier does not take the launch), blocks, 16-token groups per block, groups per wave}.
+ * groups per tile; 0: the launch runs in another tier), blocks, 16-token groups per block, groups per wave}.
  * epilogue: LSK_EPI_*, or 3 = K-slice partials (lsk_gemm_partial), 4 = LM head + argmax, 5 = fused qkv + RoPE +
  * KV append; af: fragment-major A.  A query only (no launch): for tests and measurement tools to know which
  * kernel configuration a token count reaches.  Part of the lsk_gemm* family above (solutions/packed.py:175-185). */

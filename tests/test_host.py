@@ -988,18 +988,37 @@ def test_measure_window_rules_of_the_two_engines():
 def test_fused_qkv_token_counts_reach_every_wide_configuration():
     """The token counts of the fused qkv GPU test reach both wide-tier tile widths (32- and 64-row tiles, ns 2 / 4)
     with one to three token groups per wave (every pair the tier instantiates for qkv) over the GQA shape and the
-    64-dim MHA shape together, by the library's own configuration rule (lsk_gemm_wide_config)."""
+    shape of 25 64-dim heads together, by the library's own configuration rule (lsk_gemm_wide_config), which counts
+    only launches that the many-token tier leaves."""
     from thesis_amd import _lsk
-    from test_kernels_gpu import FUSED_QKV_MS
+    from test_kernels_gpu import FUSED_QKV_HEADS, FUSED_QKV_MS
 
     _lsk.load()
     for heads, need in (((32, 8, 128), {(2, 1), (4, 1), (4, 2), (4, 3)}),
-                        ((8, 8, 64), {(2, 2), (2, 3), (4, 2), (4, 3)})):
+                        ((15, 5, 64), {(2, 2), (2, 3), (4, 2), (4, 3)})):
+        assert heads in FUSED_QKV_HEADS
         N = (heads[0] + 2 * heads[1]) * heads[2]
         got = {(c[0], c[3]) for c in (_lsk.gemm_wide_config(_lsk.EPI_QKV_ROPE, M, N, 1024) for M in FUSED_QKV_MS)
                if c[0]}
         assert need <= got, (heads, sorted(got))
         assert _lsk.gemm_wide_config(_lsk.EPI_QKV_ROPE, 64, N, 1024)[0] == 0       # <= 64 rows: decode tier
+
+
+def test_wide_config_is_zero_where_the_many_token_tier_takes_the_launch():
+    """lsk_gemm_wide_config answers for the launch that would run: with a fragment-major A no launch has a configuration
+    in both tiers, and with a row-major A (which the many-token tier does not read) the wide tier's stays."""
+    from thesis_amd import _lsk
+
+    both = 0
+    for epi, N, K, ks in ((_lsk.EPI_QKV_ROPE, 1536, 1024, 1), (_lsk.EPI_QKV_ROPE, 6144, 4096, 1),
+                          (_lsk.EPI_SILU_MUL, 14336, 4096, 1), (_lsk.EPI_PARTIAL, 4096, 14336, 4),
+                          (_lsk.EPI_ARGMAX, 128256, 4096, 1)):
+        for M in (100, 300, 512, 899, 900, 1200, 2100):
+            wide, deep = _lsk.gemm_wide_config(epi, M, N, K, ks), _lsk.gemm_deep_config(epi, M, N, K, ks)
+            assert not (wide[0] and deep[0]), (epi, M, N)
+            if deep[0] and epi != _lsk.EPI_QKV_ROPE:
+                both += _lsk.gemm_wide_config(epi, M, N, K, ks, af=False)[0] > 0
+    assert both >= 12
 
 
 class _ToyTokenizer:

@@ -964,21 +964,37 @@ def test_shifted_segment_metadata_equals_a_plan_at_the_actual_positions(cuda, sp
 
 
 FUSED_QKV_MS = [5, 32, 48, 64, 100, 160, 288, 600, 1200, 1600, 2000, 2100]   # wide tier: every (ns, msw) it picks for qkv
+FUSED_QKV_HEADS = [(32, 8, 128), (8, 8, 64), (15, 5, 64)]
 
 
 @pytest.mark.parametrize("M", FUSED_QKV_MS)
-@pytest.mark.parametrize("heads", [(32, 8, 128), (8, 8, 64)])
+@pytest.mark.parametrize("heads", FUSED_QKV_HEADS)
 def test_fused_qkv_rope_writes_what_the_unfused_path_writes(cuda, M, heads):
     """lsk_gemm_qkv_rope -- the qkv projection with RoPE and the KV append in its epilogue, the weight's q / k row
     groups RoPE-paired -- writes bitwise what the qkv GEMM without a K split (lsk_gemm_partial, ks = 1) followed by
     lsk_rope_append_partial writes: the rotated q, the K cache and the V cache (every other cache slot untouched),
-    in the decode tier (<= 64 rows) and in the wide tier (every tile width and groups-per-wave count it picks for
-    these shapes, up to 2100-token prefill sizes: test_fused_qkv_token_counts_reach_every_wide_configuration);
-    unpacking the paired storage gives the weight back."""
+    in the decode tier (<= 64 rows), in the wide tier (every tile width and groups-per-wave count it picks for
+    these shapes, up to 2100-token prefill sizes: test_fused_qkv_token_counts_reach_every_wide_configuration; the 25
+    heads of 64 dims are rows the many-token tier cannot take) and in the many-token tier; unpacking the paired storage
+    gives the weight back."""
+    _fused_qkv_equals_unfused(cuda, M, heads, 1024)
+
+
+@pytest.mark.parametrize("M,heads,K,groups", [(333, (32, 32, 128), 128, 4), (1250, (8, 4, 64), 384, 4),
+                                              (650, (32, 8, 128), 2048, 6), (2700, (8, 8, 64), 1536, 6),
+                                              (850, (32, 16, 128), 2048, 8), (1001, (32, 8, 128), 2048, 8)])
+def test_fused_qkv_many_token_tiles(cuda, M, heads, K, groups):
+    """The many-token tier's fused qkv at 4, 6 and 8 token groups per workgroup (asserted), ragged last groups and blocks
+    of unequal group counts, 64- and 128-dim heads: the writes of the unfused path."""
+    assert _lsk().gemm_deep_config(_lsk().EPI_QKV_ROPE, M, (heads[0] + 2 * heads[1]) * heads[2], K)[0] == groups
+    _fused_qkv_equals_unfused(cuda, M, heads, K)
+
+
+def _fused_qkv_equals_unfused(cuda, M, heads, K):
     lsk = _lsk()
     Hq, Hkv, D = heads
     g = _gen(2000 + M + D)
-    K, N, B, S = 1024, (Hq + 2 * Hkv) * D, 4, 1024
+    N, B, S = (Hq + 2 * Hkv) * D, 4, 1024
     m16 = lsk.frag_rows(M)
     a = torch.randn(m16, K, generator=g).to(BF16).to(cuda)
     af = lsk.PackedWeight(a).data                                          # fragment-major A, same values
