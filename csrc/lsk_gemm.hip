@@ -74,9 +74,9 @@ __global__ __launch_bounds__(256, (gemm_occupancy<NS, MS, EPI, CK>())) void gemm
   constexpr int NT = (EPI == LSK_EPI_SILU_MUL) ? 2 * NS : NS;
   static_assert(!AF || EPI == EPI_PARTIAL || EPI == EPI_ARGMAX || EPI == LSK_EPI_SILU_MUL || EPI == EPI_QKV,
                 "fragment-major A: split-K partial, silu-mul, LM head and the fused qkv");
-  // fused qkv, whole rotation pairs per tile: two or four row groups, or (NS = 1) eight rows of a group and the same eight
-  // of its partner in the next group (tile 2 p + h: rows 8 h .. 8 h + 7 of groups 2 p and 2 p + 1)
-  static_assert(EPI != EPI_QKV || (AF && (NS == 1 || NS % 2 == 0)), "fused qkv: fragment-major A");
+  // fused qkv, whole rotation pairs per tile: two row groups, or (NS = 1, one token group) eight rows of a group and the
+  // same eight of its partner in the next group (tile 2 p + h: rows 8 h .. 8 h + 7 of groups 2 p and 2 p + 1)
+  static_assert(EPI != EPI_QKV || (AF && (NS == 2 || (NS == 1 && MS == 1))), "fused qkv: tiles of rotation pairs");
   constexpr bool HALF = EPI == EPI_QKV && NS == 1;
   constexpr int E = NT * MS * 256;  // partial-sum floats per wave
   __shared__ __attribute__((aligned(16))) float red[4 * E];
@@ -887,9 +887,9 @@ static void launch_bf16(int epi, dim3 grid, hipStream_t s, const uint16_t* A, lo
 }
 
 // Fragment-major A: split-K partials, silu-mul (C row-major, or fragment-major with c_nks > 0), the LM head and
-// the fused qkv + RoPE + KV append.
+// the fused qkv + RoPE + KV append.  False: no kernel of this tile and epilogue.
 template <int NS, int MS>
-static void launch_bf16_af(int epi, dim3 grid, hipStream_t s, const uint16_t* A, const uint16_t* W, long ldw,
+static bool launch_bf16_af(int epi, dim3 grid, hipStream_t s, const uint16_t* A, const uint16_t* W, long ldw,
                            uint16_t* C, long ldc, int c_nks, float* P, float* av, int* ai, int M, int N, int K, int ffn,
                            int kslice, int nt, int mt, int m_lo, const QkvRope& qa) {
   if (epi == LSK_EPI_SILU_MUL)
@@ -903,14 +903,17 @@ static void launch_bf16_af(int epi, dim3 grid, hipStream_t s, const uint16_t* A,
     if constexpr (NS == 2 || (NS == 1 && MS == 1))
       gemm_bf16_kernel<NS, MS, EPI_QKV, gemm_unit<NS, MS, EPI_QKV>(), true><<<grid, 256, 0, s>>>(
           A, 0, W, ldw, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, M, N, K, 0, kslice, nt, mt, m_lo, 0, qa);
+    else
+      return false;
   } else
     gemm_bf16_kernel<NS, MS, EPI_PARTIAL, gemm_unit<NS, MS, EPI_PARTIAL>(), true><<<grid, 256, 0, s>>>(
         A, 0, W, ldw, nullptr, 0, nullptr, 0, P, nullptr, nullptr, M, N, K, 0, kslice, nt, mt, m_lo, 0, QkvRope{});
+  return true;
 }
 
-// Launch over nt row tiles x mt token tiles x ks K slices (the tile mapping is in the kernel).  af: a split-K
-// partial launch with a fragment-major A.
-static void dispatch_bf16(int ns, int ms, int epi, int nt, int mt, int ks, hipStream_t s, const void* A, long lda,
+// Launch over nt row tiles x mt token tiles x ks K slices (the tile mapping is in the kernel).  af: a fragment-major A.
+// A tile without a kernel is an error, never a launch left out.
+static int dispatch_bf16(int ns, int ms, int epi, int nt, int mt, int ks, hipStream_t s, const void* A, long lda,
                           const void* W, long ldw, void* C, long ldc, const void* R, long ldr, float* P, float* av,
                           int* ai, int M, int N, int K, int ffn, int kslice, bool af = false, int m_lo = 0,
                           int c_nks = 0, const QkvRope& qa = QkvRope{}) {
@@ -919,10 +922,12 @@ static void dispatch_bf16(int ns, int ms, int epi, int nt, int mt, int ks, hipSt
   const uint16_t* w = (const uint16_t*)W;
   uint16_t* c = (uint16_t*)C;
   const uint16_t* r = (const uint16_t*)R;
+  bool launched = false;
 #define LSK_GEMM_CASE(NS_, MS_)                                                                                  \
   if (ns == NS_ && ms == MS_) {                                                                                  \
+    launched = true;                                                                                             \
     if (af)                                                                                                      \
-      launch_bf16_af<NS_, MS_>(epi, grid, s, a, w, ldw, c, ldc, c_nks, P, av, ai, M, N, K, ffn, kslice, nt, mt, m_lo, qa); \
+      launched = launch_bf16_af<NS_, MS_>(epi, grid, s, a, w, ldw, c, ldc, c_nks, P, av, ai, M, N, K, ffn, kslice, nt, mt, m_lo, qa); \
     else                                                                                                         \
       launch_bf16<NS_, MS_>(epi, grid, s, a, lda, w, ldw, c, ldc, r, ldr, P, av, ai, M, N, K, ffn, kslice, nt, mt, \
                             m_lo);                                                                               \
@@ -931,6 +936,8 @@ static void dispatch_bf16(int ns, int ms, int epi, int nt, int mt, int ks, hipSt
   LSK_GEMM_CASE(2, 1) LSK_GEMM_CASE(2, 2) LSK_GEMM_CASE(2, 3) LSK_GEMM_CASE(2, 4)
   LSK_GEMM_CASE(4, 1) LSK_GEMM_CASE(4, 2) LSK_GEMM_CASE(4, 3) LSK_GEMM_CASE(4, 4)
 #undef LSK_GEMM_CASE
+  LSK_REQUIRE(launched, LSK_EUNSUPPORTED, "lsk_gemm: no kernel for a tile of %d x %d groups (launch kind %d)", ns, ms, epi);
+  return 0;
 }
 
 // Wide-M tier selection.  Above 64 tokens every row goes through the wide tier in one launch.  A configuration
@@ -1208,8 +1215,9 @@ extern "C" int lsk_gemm(int dtype, const void* A, long lda, const void* W, long 
     const int mr = M - mw;
     const int ns = tile_ns(N, mr, epilogue);
     const int ms = ms_for(mr);
-    dispatch_bf16(ns, ms, epilogue, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, lda, W, ldw, C, ldc, R, ldr,
-                  nullptr, nullptr, nullptr, M, N, K, ffn, K, false, mw);
+    const int rc = dispatch_bf16(ns, ms, epilogue, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, lda, W, ldw, C,
+                                 ldc, R, ldr, nullptr, nullptr, nullptr, M, N, K, ffn, K, false, mw);
+    if (rc) return rc;
     return lsk_check_launch("lsk_gemm(bf16)");
   }
   if (dtype == LSK_DTYPE_F32) {
@@ -1242,8 +1250,10 @@ extern "C" int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw
   const int mr = M - mw;
   const int ns = tile_ns(N, mr, EPI_PARTIAL, K / ks, ks);
   const int ms = ms_for(mr);
-  dispatch_bf16(ns, ms, EPI_PARTIAL, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), ks, (hipStream_t)stream, A, lda, W,
-                ldw, nullptr, 0, nullptr, 0, P, nullptr, nullptr, M, N, K, 0, K / ks, false, mw);
+  const int rc = dispatch_bf16(ns, ms, EPI_PARTIAL, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), ks,
+                               (hipStream_t)stream, A, lda, W, ldw, nullptr, 0, nullptr, 0, P, nullptr, nullptr, M, N, K,
+                               0, K / ks, false, mw);
+  if (rc) return rc;
   return lsk_check_launch("lsk_gemm_partial");
 }
 
@@ -1251,22 +1261,22 @@ extern "C" int lsk_gemm_partial(const void* A, long lda, const void* W, long ldw
 // rows the wide tier takes its full token blocks and the decode kernel the rest, exactly as lsk_gemm / lsk_gemm_partial
 // / lsk_head_argmax split a row-major A, with the same tiles.  The same sums in all three.  c_nks > 0 (silu-mul): C
 // fragment-major too.
-static void gemm_af(int epi, hipStream_t s, const void* A, const void* W, void* C, long ldc, int c_nks, float* P,
+static int gemm_af(int epi, hipStream_t s, const void* A, const void* W, void* C, long ldc, int c_nks, float* P,
                     float* av, int* ai, int M, int N, int K, int ffn, int ks) {
   const DeepCfg deep = deep_plan(epi, M, N, K, ks, c_stores4(C, c_nks > 0 ? 0 : ldc));
   if (deep.mg > 0) {
     lsk_gemm_deep(deep, epi, s, (const uint16_t*)A, (const uint16_t*)W, (uint16_t*)C, ldc, c_nks, nullptr, P, av, ai, M, N,
                   K, ffn, ks, QkvRope{});
-    return;
+    return 0;
   }
   const int mw = launch_wide(epi, s, (const uint16_t*)A, 0, (const uint16_t*)W, (uint16_t*)C, ldc, nullptr, 0, P, av,
                              ai, M, N, K, ffn, ks, true, c_nks);
-  if (mw == M) return;
+  if (mw == M) return 0;
   const int mr = M - mw;
   const int ms = ms_for(mr);
   const int ns = epi == EPI_PARTIAL ? tile_ns(N, mr, EPI_PARTIAL, K / ks, ks, 48) : (epi == EPI_ARGMAX ? 4 : tile_ns(N, mr, epi));
-  dispatch_bf16(ns, ms, epi, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), ks, s, A, 0, W, K, C, ldc, nullptr, 0, P,
-                av, ai, M, N, K, ffn, K / ks, true, mw, c_nks);
+  return dispatch_bf16(ns, ms, epi, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), ks, s, A, 0, W, K, C, ldc, nullptr, 0,
+                       P, av, ai, M, N, K, ffn, K / ks, true, mw, c_nks);
 }
 
 int lsk_gemm_partial_af(const void* A, const void* W, float* P, int M, int N, int K, int ks, void* stream) {
@@ -1274,7 +1284,8 @@ int lsk_gemm_partial_af(const void* A, const void* W, float* P, int M, int N, in
   LSK_REQUIRE(M >= 0 && N > 0 && N % 16 == 0 && K > 0 && ks >= 1 && K % ks == 0 && (K / ks) % 32 == 0, LSK_ESHAPE,
               "lsk_gemm_partial_af: bad shape M=%d N=%d K=%d ks=%d", M, N, K, ks);
   if (M == 0) return 0;
-  gemm_af(EPI_PARTIAL, (hipStream_t)stream, A, W, nullptr, 0, 0, P, nullptr, nullptr, M, N, K, 0, ks);
+  const int rc = gemm_af(EPI_PARTIAL, (hipStream_t)stream, A, W, nullptr, 0, 0, P, nullptr, nullptr, M, N, K, 0, ks);
+  if (rc) return rc;
   return lsk_check_launch("lsk_gemm_partial_af");
 }
 
@@ -1283,8 +1294,9 @@ int lsk_gemm_silu_af(const void* A, const void* W, void* H, int h_frag, int M, i
   LSK_REQUIRE(M >= 0 && ffn > 0 && ffn % 32 == 0 && K > 0 && K % 32 == 0, LSK_ESHAPE,
               "lsk_gemm_silu_af: bad shape M=%d ffn=%d K=%d", M, ffn, K);
   if (M == 0) return 0;
-  gemm_af(LSK_EPI_SILU_MUL, (hipStream_t)stream, A, W, H, ffn, h_frag ? ffn / 32 : 0, nullptr, nullptr, nullptr, M,
-          ffn, K, ffn, 1);
+  const int rc = gemm_af(LSK_EPI_SILU_MUL, (hipStream_t)stream, A, W, H, ffn, h_frag ? ffn / 32 : 0, nullptr, nullptr,
+                         nullptr, M, ffn, K, ffn, 1);
+  if (rc) return rc;
   return lsk_check_launch("lsk_gemm_silu_af");
 }
 
@@ -1349,8 +1361,9 @@ extern "C" int lsk_head_argmax(int dtype, const void* A, long lda, const void* W
   if (launch_wide(EPI_ARGMAX, s, (const uint16_t*)A, lda, (const uint16_t*)W, (uint16_t*)logits, ldl, nullptr, 0,
                   nullptr, av, ai, M, N, K, 0, 1) != M) {
     const int ms = ms_for(M);
-    dispatch_bf16(4, ms, EPI_ARGMAX, nt, (M + 16 * ms - 1) / (16 * ms), 1, s, A, lda, W, ldw, logits, ldl, nullptr, 0,
-                  nullptr, av, ai, M, N, K, 0, K);
+    const int rc = dispatch_bf16(4, ms, EPI_ARGMAX, nt, (M + 16 * ms - 1) / (16 * ms), 1, s, A, lda, W, ldw, logits, ldl,
+                                 nullptr, 0, nullptr, av, ai, M, N, K, 0, K);
+    if (rc) return rc;
   }
   int rc = lsk_check_launch("lsk_head_argmax(gemm)");
   if (rc) return rc;
@@ -1388,7 +1401,8 @@ extern "C" int lsk_head_norm_argmax(int dtype, const void* h, long ldh, const vo
   const size_t half = lsk_align_up((size_t)M * nt * 4, 256);
   float* av = (float*)hw;
   int* ai = (int*)(hw + half);
-  gemm_af(EPI_ARGMAX, s, xn, W, logits, ldl, 0, nullptr, av, ai, M, N, K, 0, 1);
+  rc = gemm_af(EPI_ARGMAX, s, xn, W, logits, ldl, 0, nullptr, av, ai, M, N, K, 0, 1);
+  if (rc) return rc;
   rc = lsk_check_launch("lsk_head_norm_argmax(gemm)");
   if (rc) return rc;
   argmax_tiles_kernel<<<M, 256, 0, s>>>(av, ai, nt, out, dst_idx);
@@ -1487,8 +1501,9 @@ extern "C" int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_head
     // 16.1; 384: within 3 %).  Cold weights, graph-timed.
     const int ns = N / 16 <= 256 && mr <= 16 ? 1 : 2;
     while (ms > 1 && (long)(N / 32) * ((mr + 16 * ms - 1) / (16 * ms)) < 192) --ms;
-    dispatch_bf16(ns, ms, EPI_QKV, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, 0, W, K, nullptr, 0, nullptr, 0,
-                  nullptr, nullptr, nullptr, M, N, K, 0, K, true, mw, 0, qa);
+    rc = dispatch_bf16(ns, ms, EPI_QKV, N / (16 * ns), (mr + 16 * ms - 1) / (16 * ms), 1, s, A, 0, W, K, nullptr, 0,
+                       nullptr, 0, nullptr, nullptr, nullptr, M, N, K, 0, K, true, mw, 0, qa);
+    if (rc) return rc;
   }
   return lsk_check_launch("lsk_gemm_qkv_rope");
 }

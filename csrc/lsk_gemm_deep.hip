@@ -155,7 +155,8 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
     return x;
   };
   const int s_end = s_first + sl;
-  // byte offset of a chunk's first k-step within a row group's fragments; past the last chunk: the last one's again
+  // byte offset of a chunk's first k-step within a row group's fragments; past the last chunk (the loads that run ahead
+  // of the loop's end): a chunk of the last slice again, loaded and never multiplied
   auto kofs = [&](const Seq& x) { return (unsigned)((min(x.s, s_end - 1) * (kslice >> 5)) + x.c * 4) * 1024u; };
 
   auto load_w = [&](lsk_bf16x8 (&w)[NG], unsigned ko, int ksi) {
