@@ -646,6 +646,9 @@ def test_rocprof_summary_counts_after_the_calibration_copy(tmp_path, capsys):
     # the fragment-major-activation flag is a bool template argument
     assert ps.classify("gemm_bf16_kernel<2, 2, 3, 4, true>", 192 * 256) == "gemm_qkv"
     assert ps.classify("gemm_bf16_kernel<4, 3, 2, 2, false>") == "gemm_w13"
+    # the many-token tier: token groups, then the epilogue
+    for epi, cls in ((1, "gemm_o_w2"), (2, "gemm_w13"), (3, "gemm_qkv_o_w2"), (4, "gemm_lm_head"), (5, "gemm_qkv")):
+        assert ps.classify(f"gemm_deep_kernel<8, {epi}>", 512 * 256) == cls
 
 
 def test_method_registry():

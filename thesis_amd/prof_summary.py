@@ -66,6 +66,10 @@ def classify(short: str, grid_x_threads=None) -> str:
     if m:                                    # wide-M tier: same classes, qkv and o / w2 not told apart
         cls = _EPI.get(m.group(3), "gemm")
         return "gemm_qkv_o_w2" if cls == "gemm_partial" else cls
+    m = re.match(r"gemm_deep_kernel<(\d+), (\d+)>", short)
+    if m:                                    # many-token tier: as the wide tier; its residual launches are o and w2
+        cls = _EPI.get(m.group(2), "gemm")
+        return {"gemm_partial": "gemm_qkv_o_w2", "gemm_residual": "gemm_o_w2"}.get(cls, cls)
     for key, cls in (("attn_bf16_kernel", "attention"), ("attn_f32_kernel", "attention"),
                      ("attn_combine_kernel", "attention_combine"), ("add_rmsnorm_kernel", "rmsnorm"),
                      ("rope_append_kernel", "rope_append"), ("argmax_tiles_kernel", "head_pick"),
