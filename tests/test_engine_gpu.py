@@ -572,3 +572,43 @@ def test_launch_ahead_shallow_segments_change_no_token(cuda, dtype, forced):
     ahead, eng, _ = _run_gpu(g, prompts, 3, 30, launch_ahead=True, **kw)
     assert ahead == plain
     assert eng.ahead_used > 0
+
+
+def test_long_segment_equals_the_same_tokens_in_short_pieces(cuda):
+    """One segment of 1150 tokens, whose o and w2 launches sum their K slices and write the residual stream themselves
+    (asserted), against the same tokens in pieces of at most 64 (decode tier, K-slice partials added by the next norm):
+    the hidden states, the exit hiddens of every layer and the K / V caches are bitwise equal."""
+    from thesis_amd import _lsk
+    from thesis_amd.common.model import LayerSkipLlama, ModelConfig
+    from thesis_amd.solutions.packed import Block, build_packed, packed_layers
+
+    cfg = ModelConfig(vocab_size=64, dim=2048, n_layers=3, n_heads=16, n_kv_heads=4, head_dim=128, intermediate_size=2048,
+                      rope_theta=10000.0, max_position_embeddings=2048)
+    long, short = 1113, 37
+    N = long + short
+    for K in (cfg.n_heads * cfg.head_dim, cfg.intermediate_size):
+        assert _lsk.gemm_deep_config(_lsk.EPI_RESIDUAL, N, cfg.dim, K, _lsk.gemm_plan(cfg.dim, K)[1])[0] > 0
+    g = torch.Generator(device=cuda).manual_seed(3)
+    x = torch.randn(N, cfg.dim, generator=g, device=cuda).to(torch.bfloat16)       # packed order: the short block first
+    res = []
+    for piece in (None, 64):
+        m = LayerSkipLlama.random(cfg, seed=1, device=cuda, max_seq=2048)
+        m.allocate_cache(2, 1216)
+        for kv in (*m.cache.kstore, *m.cache.vb):
+            kv.zero_()
+        if piece is None:
+            calls = [([Block(0, 0, long), Block(1, 0, short)], x)]
+        else:
+            calls = [([Block(1, 0, short)], x[:short])]
+            calls += [([Block(0, p, min(piece, long - p))], x[short + p:short + min(p + piece, long)])
+                      for p in range(0, long, piece)]
+        outs = []
+        for blocks, xs in calls:
+            cap = {}
+            h = packed_layers(m, xs, build_packed(m, blocks), 0, 3, cap, (1, 2, 3))
+            outs.append([h, cap[1], cap[2], cap[3]])
+        res.append([torch.cat(t) for t in zip(*outs)] + [*m.cache.kstore, *m.cache.vb])
+    assert all(torch.isfinite(t).all() and (t != 0).any() for t in res[0][:4])
+    assert not torch.equal(res[0][1], res[0][2])
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
