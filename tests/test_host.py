@@ -507,6 +507,29 @@ def test_linear_fit_recovers_planted_coefficients():
     assert s["m_n64_256"]["n"] == 1 and "m_prefill" not in s
 
 
+@pytest.mark.parametrize("bf16", [True, False])
+def test_flops_eff_launches_the_gemms_as_the_layer_does(monkeypatch, bf16):
+    """The layer runner reads fragment-major activations: o at every token count, w13 and w2 above 64 tokens (where the
+    wide and the many-token tier run); F_eff times those launches.  fp32 layers are row-major throughout."""
+    from thesis_amd import _lsk
+    from thesis_amd.solutions import calibrate as cal
+
+    calls = []
+    monkeypatch.setattr(cal, "timed_ms", lambda fn: (fn(), 1.0)[1])
+    for name in ("gemm", "gemm_partial", "gemm_partial_frag", "gemm_silu_frag", "gemm_qkv_rope"):
+        monkeypatch.setattr(_lsk, name, lambda *a, _n=name, **k: calls.append(_n))
+    weight = lambda n, k, heads=None: SimpleNamespace(shape=(n, k), qkv_heads=heads)   # noqa: E731
+    lw = SimpleNamespace(wqkv=weight(256, 128, (2, 1, 64) if bf16 else None), wo=weight(128, 128), w13=weight(512, 128),
+                         w2=weight(128, 256))
+    m = SimpleNamespace(layers=[lw], device="cpu", dtype=torch.bfloat16 if bf16 else torch.float32, q_size=128,
+                        rope_cos=None, rope_sin=None,
+                        cfg=SimpleNamespace(dim=128, intermediate_size=256, n_heads=2, n_kv_heads=1, head_dim=64))
+    assert cal.measure_flops_eff(m, (32, 64, 65, 512))["flops_eff_at_n"] == 512
+    few = ["gemm_qkv_rope", "gemm_partial_frag", "gemm", "gemm_partial"]
+    many = ["gemm_qkv_rope", "gemm_partial_frag", "gemm_silu_frag", "gemm_partial_frag"]
+    assert calls == (2 * few + 2 * many if bf16 else 16 * ["gemm"])
+
+
 def test_calibration_record_loads_as_cost_models(tmp_path):
     from thesis_amd.common.model import PRESETS
     from thesis_amd.solutions.cost_model import (GPUParams, LinearCostModel, RooflineCostModel, load_cost_model,

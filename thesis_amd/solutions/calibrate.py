@@ -9,8 +9,9 @@ Measured, each with HIP events on the stream liblsk launches on (median of repet
              (solutions/calibrate.py:59-62)
   flops      8192^3 bf16 matmul through torch (hipBLASLt): the device's dense rate as a library reaches
              it, kept only for the roofline-peak variant (solutions/calibrate.py:63-66)
-  flops_eff  highest flop rate of the model's own layer GEMMs as the layer runs them (qkv, o, w2 as K-slice
-             partials, w13 + silu-mul) for n = 1..512 tokens (solutions/calibrate.py:126-140)
+  flops_eff  highest flop rate of the model's own layer GEMMs as the layer runs them (qkv + RoPE + append, o and w2
+             as K-slice partials, w13 + silu-mul, in its input layouts) for n = 1..512 tokens
+             (solutions/calibrate.py:126-140)
   knee       hinge fit t = a + b max(n - knee, 0) of one real packed layer timed for n = 1..512
              single-token requests (solutions/calibrate.py:143-172)
   t_op       back-to-back tiny liblsk launches (a one-row lsk_copy_rows) (solutions/calibrate.py:67-72)
@@ -116,52 +117,72 @@ def trace_ops(m) -> dict:
 
 
 def _layer_gemms(m) -> list:
-    """(weight, input width, K slices) of the four projections of layer 0 as the bf16 layer runner launches
-    them: qkv fused with RoPE + append (-1), o and w2 as K-slice partials (the plan's slice count), w13 with the
-    silu-mul epilogue (0)."""
+    """(name, weight, input width, K slices) of the four projections of layer 0: o and w2 as K-slice partials (the plan's
+    slice count), qkv fused with RoPE + append and w13 with the silu-mul epilogue unsplit."""
     lw, c = m.layers[0], m.cfg
-    out = []
-    for w, k in ((lw.wqkv, c.dim), (lw.wo, m.q_size), (lw.w13, c.dim), (lw.w2, c.intermediate_size)):
-        if w is lw.wqkv and getattr(w, "qkv_heads", None) is not None:
-            ks = -1
+    bf16 = m.dtype == torch.bfloat16
+    return [(name, w, k, _lsk.gemm_plan(w.shape[0], k)[1] if bf16 and split else 1)
+            for name, w, k, split in (("qkv", lw.wqkv, c.dim, False), ("o", lw.wo, m.q_size, True),
+                                      ("w13", lw.w13, c.dim, False), ("w2", lw.w2, c.intermediate_size, True))]
+
+
+def _layer_launches(m, n: int, kv) -> list:
+    """The projections' launches of n tokens in the layer runner's input layouts: bf16 fragment-major for qkv and o, and for
+    w13 and w2 above one GEMM token tile; row-major otherwise and in fp32.  kv: scratch (K, V, rows, positions)."""
+    c, frag = m.cfg, {"qkv", "o"}
+    if n > _lsk.GEMM_TOKEN_TILE and c.dim % 32 == 0 and c.intermediate_size % 64 == 0:
+        frag |= {"w13", "w2"}
+    calls = []
+    for name, w, k, ks in _layer_gemms(m):
+        N = w.shape[0]
+        if m.dtype != torch.bfloat16:
+            x = torch.randn(n, k, device=m.device, dtype=m.dtype)
+            out = torch.empty(n, N // 2 if name == "w13" else N, device=m.device, dtype=m.dtype)
+            epi = _lsk.EPI_SILU_MUL if name == "w13" else _lsk.EPI_NONE
+            calls.append(lambda x=x, w=w, out=out, epi=epi: _lsk.gemm(x, w, out=out, epilogue=epi))
+            continue
+        x = torch.randn(_lsk.frag_rows(n) * k, device=m.device, dtype=m.dtype)
+        if name not in frag:
+            x = x[:n * k].view(n, k)
+        if name == "qkv":
+            q = torch.empty(n, c.n_heads, c.head_dim, device=m.device, dtype=m.dtype)
+            kc, vc, rows, pos = kv
+            calls.append(lambda x=x, w=w, q=q: _lsk.gemm_qkv_rope(x, w, n, q, kc, vc, m.rope_cos, m.rope_sin, rows[:n],
+                                                                  pos[:n]))
+        elif name == "w13":
+            h = torch.empty(_lsk.frag_rows(n) * (N // 2), device=m.device, dtype=m.dtype)
+            if name in frag:
+                calls.append(lambda x=x, w=w, h=h: _lsk.gemm_silu_frag(x, n, w, h, True))
+            else:
+                h = h[:n * (N // 2)].view(n, N // 2)
+                calls.append(lambda x=x, w=w, h=h: _lsk.gemm(x, w, out=h, epilogue=_lsk.EPI_SILU_MUL))
         else:
-            ks = 0 if w is lw.w13 else (_lsk.gemm_plan(w.shape[0], k)[1] if m.dtype == torch.bfloat16 else 1)
-        out.append((w, k, ks))
-    return out
+            P = torch.empty(ks, n, N, device=m.device)
+            if name in frag:
+                calls.append(lambda x=x, w=w, P=P, ks=ks: _lsk.gemm_partial_frag(x, n, w, ks, out=P))
+            else:
+                calls.append(lambda x=x, w=w, P=P, ks=ks: _lsk.gemm_partial(x, w, ks, out=P))
+    return calls
 
 
 def measure_flops_eff(m, ns=N_GRID) -> dict:
-    """F_eff: the highest flop rate the model's own layer GEMMs reach for n = 1..512 tokens.  At small n
-    they stream the weights (rate grows with n); past the ridge they are MFMA-bound."""
-    shapes = _layer_gemms(m)
-    params = sum(w.shape[0] * w.shape[1] for w, _, _ in shapes)
-    rows = []
-    c = m.cfg
-    if any(ks < 0 for _, _, ks in shapes):           # scratch cache row for the fused qkv launch (positions 0 .. n-1)
+    """F_eff: the highest flop rate the model's own layer GEMMs reach for n = 1..512 tokens, launched as the layer runner
+    launches them.  At small n they stream the weights (rate grows with n); past the ridge they are MFMA-bound."""
+    params = sum(w.shape[0] * w.shape[1] for _, w, _, _ in _layer_gemms(m))
+    rows, c, kv = [], m.cfg, None
+    if m.dtype == torch.bfloat16:                    # scratch cache row for the fused qkv launch (positions 0 .. n-1)
         s_kv = (max(ns) + 31) // 32 * 32
-        kc = torch.zeros(1, c.n_kv_heads, s_kv // 32, c.head_dim // 16, 64, 8, dtype=m.dtype, device=m.device)
-        vc = torch.zeros(1, c.n_kv_heads, s_kv // 32, c.head_dim, 32, dtype=m.dtype, device=m.device)
-        rows_s = torch.zeros(max(ns), dtype=torch.int32, device=m.device)
-        pos_s = torch.arange(max(ns), dtype=torch.int32, device=m.device)
+        kv = (torch.zeros(1, c.n_kv_heads, s_kv // 32, c.head_dim // 16, 64, 8, dtype=m.dtype, device=m.device),
+              torch.zeros(1, c.n_kv_heads, s_kv // 32, c.head_dim, 32, dtype=m.dtype, device=m.device),
+              torch.zeros(max(ns), dtype=torch.int32, device=m.device),
+              torch.arange(max(ns), dtype=torch.int32, device=m.device))
     with torch.inference_mode():
         for n in ns:
-            xs = [torch.randn(_lsk.frag_rows(n) * k if ks < 0 else n * k, device=m.device, dtype=m.dtype).view(
-                -1 if ks < 0 else n, *(() if ks < 0 else (k,))) for _, k, ks in shapes]
-            outs = [torch.empty(n, c.n_heads, c.head_dim, device=m.device, dtype=m.dtype) if ks < 0 else
-                    torch.empty(n, w.shape[0] // 2, device=m.device, dtype=m.dtype) if ks == 0 else
-                    (torch.empty(ks, n, w.shape[0], device=m.device) if m.dtype == torch.bfloat16 else
-                     torch.empty(n, w.shape[0], device=m.device, dtype=m.dtype)) for w, _, ks in shapes]
+            calls = _layer_launches(m, n, kv)
 
             def run():
-                for (w, _, ks), x, o in zip(shapes, xs, outs):
-                    if ks < 0:
-                        _lsk.gemm_qkv_rope(x, w, n, o, kc, vc, m.rope_cos, m.rope_sin, rows_s[:n], pos_s[:n])
-                    elif ks == 0:
-                        _lsk.gemm(x, w, out=o, epilogue=_lsk.EPI_SILU_MUL)
-                    elif m.dtype == torch.bfloat16:
-                        _lsk.gemm_partial(x, w, ks, out=o)
-                    else:
-                        _lsk.gemm(x, w, out=o)
+                for f in calls:
+                    f()
             ms = timed_ms(run)
             rows.append({"n": n, "ms": ms, "flop_per_ms": 2.0 * params * n / ms})
     best = max(rows, key=lambda r: r["flop_per_ms"])
