@@ -1030,13 +1030,15 @@ static WideCfg wide_plan(int epi, int M, int N, int K, int ks, bool af, bool c_o
 }
 
 // The wide tier's estimated time (us) of a launch it takes: its cost fitted to measurements over the presets' projections
-// (within 25 %; the presets' heads and launches of two or more rounds scatter most).
+// (within 25 %, launches of two or more rounds scatter most) and, for the head, over 4096 to 128256 rows of 512 to 4096 (its
+// logits are a large part where K is small; within 6 %, at most 21 %).
 static double wide_us(int epi, int M, int N, int K, int ks) {
   double cost = 0.0;
   wide_config(epi, M, N, ks, &cost);
   cost *= (double)(K / ks) / 4096.0;
   if (epi == LSK_EPI_SILU_MUL) return 15.8 * cost + 9.0;
   if (epi == EPI_PARTIAL) return 7.4 * cost + 4.5 + 2.0 * ks * (double)M * N * 4.0 / 4.5e6;
+  if (epi == EPI_ARGMAX) return 7.6 * cost + 3.5 + 3.55 * (double)M * N * 2.0 / 4.5e6;
   return 11.1 * cost + 4.5;
 }
 
@@ -1051,8 +1053,10 @@ static double wide_us(int epi, int M, int N, int K, int ks) {
 //   preset shapes, two within 4 %); partials where its estimate is the lower one (512 x 512 at 1517: 17.2 against 19.8,
 //   the presets' 11 % slower to 61 % faster); silu-mul up to 1.15 times the wide tier's estimate, which is the low one
 //   where it plans two rounds (1408 x 2048 at 900: 22.8 against 28.4 us, left to the wide tier; at 2100: 83.6 against 35.4).
-// * From LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's.  8B shape at 304 / 512 rows: qkv
-//   54.6 / 55.5 us against the wide tier's 46.7 / 58.2, w13 116 / 144 against 108 / 174, w2 74 / 82 against 62 / 97.
+// * From LSK_DEEP_MIN_TOKENS on where its estimate is 10-15 % below the wide tier's (the head's, which scatter less: where
+//   it is the lower one).  8B shape at 304 / 512 rows: qkv 54.6 / 55.5 us against the wide tier's 46.7 / 58.2, w13 116 / 144
+//   against 108 / 174, w2 74 / 82 against 62 / 97, head 446 / 562 against 453 / 719; 7B head at 304 rows 129 against 125.
+//   (Of 91 head launches at 256-899 rows, 4096-128256 x 512-4096, none is picked more than 1.1 % slower.)
 static DeepCfg deep_plan(int epi, int M, int N, int K, int ks, bool c_ok) {
   const DeepCfg none{0, 0, 0, 0.0};
   if (!c_ok) return none;
@@ -1070,7 +1074,7 @@ static DeepCfg deep_plan(int epi, int M, int N, int K, int ks, bool c_ok) {
     if (epi == EPI_QKV || epi == EPI_ARGMAX) return d;
     f = epi == EPI_PARTIAL ? 1.0 : 1.15;
   } else {
-    f = epi == EPI_PARTIAL || epi == EPI_ARGMAX ? 0.85 : 0.9;  // the partials' and the head's estimates scatter more
+    f = epi == EPI_ARGMAX ? 1.0 : (epi == EPI_PARTIAL ? 0.85 : 0.9);
   }
   return d.us < f * wide_us(epi, M, N, K, ks) ? d : none;
 }

@@ -391,10 +391,11 @@ __global__ __launch_bounds__(256, MG <= 4 ? 2 : 1) void gemm_deep_kernel(const u
 // Configuration of a launch (N: output columns, ffn for silu-mul) and its estimated time.  A workgroup of mg token groups
 // walks c chunks of 128 k; the times below are of the busiest CU, fitted to MI355X measurements over the 1B, 7B and 8B
 // projections at 256-4001 tokens:
-//   mg = 8 / 6 (one workgroup per CU): 1.7 c + 12 (a single round: 6 with partials, else 14) / 1.25 c + 13 us each (mg = 6: 1.4 c up to
-//     1024 tokens)
-//   mg = 4 (two per CU): 2.1 c + 3 us per pair (2.5 c up to 1024 tokens and with partials, 2.5 c + 8 for the LM head), a
-//     lone one 1.3 c + 10 us (1.5 c + 9 summing its slices)
+//   mg = 8 / 6 (one workgroup per CU): 1.7 c + 12 (a single round: 6 with partials, else 14) / 1.25 c + 13 us each (mg = 6:
+//     1.4 c up to 1024 tokens)
+//   mg = 4 (two per CU): 2.1 c + 3 us per pair (2.5 c up to 1024 tokens and with partials), a lone one 1.3 c + 10 us (1.5 c +
+//     9 summing its slices)
+//   the LM head, whose logits and maxima cost more per workgroup: 1.8 c + 12, 1.66 c + 10, 2.45 c + 8 and 1.4 c + 9
 // plus 3 us per slice summed, plus the stores of the partials.  Larger mg moves fewer bytes per product (24, 22 and 20 KiB
 // per k-step for 8, 6 and 4 x 16 tokens of 256 rows), smaller mg splits a segment into more workgroups and overlaps one
 // workgroup's epilogue with the other's products: w13 of the 8B shape at 4001 tokens 920 / 992 / 943 us, at 512 tokens
@@ -418,12 +419,14 @@ DeepCfg lsk_deep_plan(int epi, int M, int N, int K, int ks) {
       const double c = (double)(ks / split) * (K / ks / 128);
       double us;
       if (mg == 4) {
-        const double lone = sum ? 1.5 * c + 9.0 : 1.3 * c + 10.0;
-        const double pair = (partial || head || M <= 1024 ? 2.5 : 2.1) * c + (head ? 8.0 : 3.0) + (sum ? 2.5 * ks : 0.0);
+        const double lone = head ? 1.4 * c + 9.0 : (sum ? 1.5 * c + 9.0 : 1.3 * c + 10.0);
+        const double pair = head ? 2.45 * c + 8.0 : (partial || M <= 1024 ? 2.5 : 2.1) * c + 3.0 + (sum ? 2.5 * ks : 0.0);
         us = (n / 2) * pair + (n & 1 ? lone : 0.0);
       } else {
-        us = n * (mg == 8 ? 1.7 * c + (n > 1 ? 12.0 : (partial ? 6.0 : 14.0)) : (M <= 1024 ? 1.4 : 1.25) * c + 13.0) +
-             (sum ? 3.0 * ks * n : 0.0);
+        const double each = head ? (mg == 8 ? 1.8 * c + 12.0 : 1.66 * c + 10.0)
+                                 : (mg == 8 ? 1.7 * c + (n > 1 ? 12.0 : (partial ? 6.0 : 14.0))
+                                            : (M <= 1024 ? 1.4 : 1.25) * c + 13.0);
+        us = n * (each + (sum ? 3.0 * ks : 0.0));
       }
       if (partial) us += 1.3 * ks * slice_us;
       if (best.mg == 0 || us < best.us) best = DeepCfg{mg, mb, split, us};

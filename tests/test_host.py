@@ -1143,8 +1143,12 @@ def test_deep_tier_leaves_weights_of_few_tiles_to_the_decode_tier():
             assert lsk.gemm_deep_config(lsk.EPI_PARTIAL, M, dim, ffn, ks)[0] > 0
         assert lsk.gemm_deep_config(lsk.EPI_RESIDUAL, 1517, dim, dim, 8 if dim == 2048 else 4)[0] > 0
         assert lsk.gemm_deep_config(lsk.EPI_RESIDUAL, 4001, dim, ffn, ks)[0] > 0
-    # the 1B head at 1152 rows: 8 token groups a workgroup (746 us; 4 groups 887, the wide tier 824)
+    # the 1B head at 1152 rows: 8 token groups a workgroup (746 us; 4 groups 887, the wide tier 824); at 304 rows the tier
+    # takes the 1B and 8B heads (258 / 447 us against 275 / 467) and leaves the 7B one (132 against 128)
     assert lsk.gemm_deep_config(lsk.EPI_ARGMAX, 1152, 128256, 2048)[0] == 8
+    assert lsk.gemm_deep_config(lsk.EPI_ARGMAX, 304, 128256, 2048)[0] > 0
+    assert lsk.gemm_deep_config(lsk.EPI_ARGMAX, 304, 128256, 4096)[0] > 0
+    assert lsk.gemm_deep_config(lsk.EPI_ARGMAX, 304, 32000, 4096)[0] == 0
 
 
 @pytest.mark.parametrize("M", [512, 901])

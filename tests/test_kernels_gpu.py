@@ -808,7 +808,7 @@ MANY_TOKEN_CASES = [
     ("partial", 2700, 1536, 2048, 4, 6), ("partial", 2049, 2048, 1280, 2, 8),
     ("silu", 333, 6144, 128, 1, 4), ("silu", 400, 8192, 2048, 1, 8), ("silu", 450, 6144, 1536, 1, 6),
     ("silu", 901, 2560, 1280, 1, 6), ("silu", 1001, 3072, 2048, 1, 8), ("silu", 1250, 1024, 384, 1, 4),
-    ("head", 257, 12288, 2048, 1, 4), ("head", 600, 12288, 1024, 1, 8), ("head", 650, 6144, 2048, 1, 6),
+    ("head", 300, 12288, 1024, 1, 4), ("head", 600, 12288, 1024, 1, 8), ("head", 450, 12288, 1024, 1, 6),
     ("head", 901, 256, 128, 1, 4), ("head", 1001, 6144, 1024, 1, 8), ("head", 2700, 1536, 512, 1, 6),
     ("residual", 901, 6144, 1280, 2, 6), ("residual", 1001, 6144, 2048, 2, 8), ("residual", 1517, 768, 384, 3, 4),
     ("residual", 1517, 2048, 2048, 8, 4),
