@@ -4,9 +4,9 @@
 // stream.  The wide tier re-reads its activations from L2 for every 64 weight rows (400-800 TFLOP/s); here a workgroup of
 // four waves owns 256 weight rows (64 per wave, read straight into registers three k-steps ahead: no other wave needs
 // them) x MG 16-token groups (staged through LDS and shared by the four waves).  MG = 8 and 6 run one workgroup per CU
-// (a wave holds up to 32 tiles in two accumulator sets), MG = 4 two.  MI355X, 4001 tokens of the 8B shape: qkv
-// 366 -> 195 us, o with its norm 430 -> 180, w13 1160 -> 900 (1050 TFLOP/s; the clock falls to 1.9 GHz there), w2 with its
-// norm 1150 -> 450.
+// (a wave holds up to 32 tiles in two accumulator sets), MG = 4 two.  MI355X, 4001 tokens of the 8B shape,
+// cold weights, graph-timed (the wide tier first): qkv 403 -> 203 us, o with its norm 430 -> 188, w13 1198 -> 915 (1030
+// TFLOP/s; the clock falls to 1.9 GHz there), w2 with its norm 1155 -> 450.
 //
 // Exactly the decode kernel's sums, as the wide tier: within a K slice the chunks of 128 k are visited class by class
 // (0, 4, 8, ...; 1, 5, ...; ...), each class into a fresh accumulator `cur` that is added to the running `tot` at its end.

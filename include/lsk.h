@@ -101,7 +101,7 @@ size_t lsk_attn_workspace_bytes(int n_parts, int n_kv_heads, int head_dim);
  * V blocked-transposed [B, Hkv, S/32, D, 32], out [N, Hq*D].  scale = 1/sqrt(D) for the reference's SDPA default.
  * bf16 runs n_slots persistent workgroups over the schedule records (recs, n_rounds); rows_cap is the cap the
  * plan was made with (16: one-tile kernel, Q in registers; 32 / 48: three-tile kernel, Q in LDS); the two
- * kernels give bitwise equal outputs.  fp32 reads works.
+ * kernels give bitwise equal outputs.  fp32 reads works; its q and caches may start at any fp32 address.
  * Replaces solutions/packed.py:142-166 (_attend: per-bucket gather + masked SDPA + scatter)
  * and common/model.py:352-364 (the padded path's masked SDPA). */
 int lsk_ragged_attn(int dtype, const void* q, const void* kcache, const void* vcache, const int32_t* blocks,
@@ -208,7 +208,8 @@ int lsk_add_rmsnorm(int dtype, const void* x, long ldx, const float* partials, i
  * with apply_rope (common/model.py:143-150, solutions/packed.py:176-179) and the KV write (solutions/packed.py:
  * 180-181).  A: the normalised rows fragment-major (lsk_frag_off, ceil(M/16)*16 rows x K); W: lsk_pack_weight_qkv
  * storage.  Writes q_out [M, n_heads, head_dim] (rotated), the K cache (rotated) and the V cache at (rows[m],
- * pos[m]), with lsk_rope_append's arithmetic on rnd(the full-K sum).  head_dim % 32 == 0, max_seq % 32 == 0. */
+ * pos[m]), with lsk_rope_append's arithmetic on rnd(the full-K sum).  head_dim % 32 == 0, max_seq % 32 == 0.  q_out, the
+ * caches and the tables may start at any address that aligns their elements. */
 int lsk_gemm_qkv_rope(const void* A, const void* W, int M, int n_heads, int n_kv_heads, int head_dim, int K,
                       void* q_out, void* kcache, void* vcache, const float* cos_tab, const float* sin_tab, int tab_len,
                       const int32_t* rows, const int32_t* pos, int max_batch, int max_seq, void* stream);
