@@ -17,9 +17,10 @@ typedef __bf16 lsk_bf16x8 __attribute__((ext_vector_type(8)));
 typedef short lsk_s16x4 __attribute__((ext_vector_type(4)));
 typedef float lsk_f32x4 __attribute__((ext_vector_type(4)));
 typedef int lsk_i32x4 __attribute__((ext_vector_type(4)));
-// Memory operands of one 16- or 8-byte instruction at addresses that only their elements align (4 fp32, 4 bf16): the
+// Memory operands of one 16- or 8-byte instruction at addresses that only their elements align (4 fp32, 8 or 4 bf16): the
 // entry points ask no more of the caller's tables, fp32 caches and bf16 rows, and gfx950 takes such addresses at no cost.
 typedef float lsk_f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t lsk_u32x4_u __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t lsk_u32x2_u __attribute__((ext_vector_type(2), aligned(2)));
 
 // Word 3 of a raw buffer descriptor on gfx9-family parts (gfx950): 32-bit data format, no swizzle, no stride;

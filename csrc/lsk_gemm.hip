@@ -283,7 +283,8 @@ __global__ __launch_bounds__(256, (gemm_occupancy<NS, MS, EPI, CK>())) void gemm
         const float o1 = rbf(silu_f(rbf(reduced(a0, ml, w0 + 1)))) * rbf(reduced(a0 + NS, ml, w0 + 1));
         pk[i >> 1] = (uint32_t)f2bf(o0) | ((uint32_t)f2bf(o1) << 16);
       }
-      *(uint4*)(C + (c_nks > 0 ? lsk_frag_off(m, n, c_nks) : (long)m * ldc + n)) = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+      *(lsk_u32x4_u*)(C + (c_nks > 0 ? lsk_frag_off(m, n, c_nks) : (long)m * ldc + n)) =
+          (lsk_u32x4_u){pk[0], pk[1], pk[2], pk[3]};
     }
   } else {
     for (int o = tid; o < TN * TM; o += 256) {
@@ -1010,7 +1011,7 @@ static void launch_wide_kernel(dim3 grid, hipStream_t s, bool af, const uint16_t
 
 // Whether a bf16 output takes 4-element stores: whole 8-byte rows from an 8-byte aligned base (no output: nothing to
 // store).  The wide and the many-token tier store 4 elements at a time; any other output (the head accepts every row
-// stride >= N) is the decode kernel's, which stores single elements.
+// stride >= N) is the decode kernel's, whose stores take any address.
 static bool c_stores4(const void* C, long ldc) { return C == nullptr || (ldc % 4 == 0 && (uintptr_t)C % 8 == 0); }
 
 // Whether the wide tier takes a launch (ns == 0: no) and its configuration.  c_ok: c_stores4 of the output.

@@ -913,6 +913,22 @@ def test_head_logits_rows_of_any_stride_and_base(cuda, M, pad, first):
     assert (buf[:, :first] == 7.0).all() and (buf[:, first + N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("M", [8, 40, 100])
+def test_gemm_outputs_at_any_bf16_address(cuda, M):
+    """Outputs one and four elements past a 16-byte boundary, in the decode and the wide tier: the aligned bits."""
+    lsk = _lsk()
+    N, K = 8192, 128
+    g = _gen(M)
+    a, r = torch.randn(M, K, generator=g).to(BF16).to(cuda), torch.randn(M, N, generator=g).to(BF16).to(cuda)
+    w = lsk.PackedWeight((torch.randn(2 * N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    h = lsk.PackedWeight((torch.randn(N, K, generator=g) * 0.05).to(BF16).to(cuda))
+    for wt, kw in ((w, {"epilogue": lsk.EPI_SILU_MUL}), (h, {}), (h, {"epilogue": lsk.EPI_RESIDUAL, "residual": r})):
+        want = lsk.gemm(a, wt, **kw)
+        for by in (1, 4):
+            out = _shifted(torch.zeros(M, N, dtype=BF16, device=cuda), by)
+            assert torch.equal(lsk.gemm(a, wt, out=out, **kw), want), (by, kw)
+
+
 @pytest.mark.parametrize("split", [4096, 128])
 def test_shifted_segment_metadata_equals_a_plan_at_the_actual_positions(cuda, split):
     """A decode segment planned at its verifiers' upper-bound positions (all drafts accepted) and moved back on the
